@@ -25,7 +25,8 @@ struct orn_device_scene {
     orn_ctx *ctx;
     orn::DevScene ds;
     std::vector<void *> allocations;
-    uint32_t stack_slots;   // BVH2 traversal
+    uint32_t stack_slots;   // BVH2 traversal in the reference's order
+    uint32_t traversal_slots;  // BVH2 launches: the larger of that and the search tree's
     uint32_t stack_slots4;  // BVH4 traversal
     uint32_t trace_width;   // node width orn_trace_rays uses
     uint32_t features;      // SceneFeatures present in the arrays

@@ -1813,7 +1813,7 @@ orn_status enqueue_render(orn_nrc *n, orn_target *t, const orn_constant_params *
         n->tile_count = tiles;
     }
     DevScene ds = s->ds;
-    ds.stack_slots = s->stack_slots;
+    ds.stack_slots = s->traversal_slots;
     const size_t lds = size_t(ds.stack_slots) * kBlock * sizeof(uint32_t);
     float cur = params->current_iteration;
     const uint32_t iters = std::max(iterations, 1u);
@@ -1847,7 +1847,7 @@ orn_status enqueue_train_paths(orn_nrc *n, const orn_constant_params *params, ui
 {
     orn_device_scene *s = n->scene;
     DevScene ds = s->ds;
-    ds.stack_slots = s->stack_slots;
+    ds.stack_slots = s->traversal_slots;
     const size_t lds = size_t(ds.stack_slots) * kBlock * sizeof(uint32_t);
     nrc_reset_count_kernel<<<1, 64, 0, st>>>(n->counters + 1);
     if (n->cfg.train_paths) ORN_NRC_DISPATCH(launch_train_paths, s->features, n, ds, *params, frame, st, lds);

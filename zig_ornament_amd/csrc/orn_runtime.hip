@@ -30,6 +30,7 @@
 
 #include "../../include/ornament_hip.h"
 #include "orn_handles.h"
+#include "orn_sah.h"
 #include "orn_trace.h"
 
 using namespace orn;
@@ -52,7 +53,7 @@ struct KernelParams {
     uint32_t regroup;       // waiting lanes that trigger a shading round
     uint32_t leaf_regroup;  // lanes at a leaf that trigger a leaf round
     uint32_t node_steps;    // internal nodes per lane between round checks
-    uint32_t root;          // TLAS root reference (single image)
+    uint32_t root;          // TLAS root reference rays start from (single image)
     uint32_t chunk;         // samples per job of a split pixel (single image)
     uint32_t chunks;        // jobs per split pixel (single image)
     uint32_t epoch;         // tag of this launch in the stage words (single image)
@@ -69,13 +70,15 @@ struct BatchItem {
     uint32_t iterations;
     uint32_t tiles_x;
     uint32_t px_base;   // first pixel of the image in the pooled buffers
-    uint32_t root;      // TLAS root reference of the image's scene
+    uint32_t root;      // TLAS root reference rays start from
     uint32_t tex_base;  // first texture of the image's scene in the shared table
     uint32_t chunk;     // samples per job of a split pixel
     uint32_t chunks;    // jobs per split pixel
     uint32_t epoch;     // tag of this launch in the stage words
+    uint32_t root2;     // TLAS root of the reference's order (rays searched again)
+    uint32_t pad[3];
 };
-static_assert(sizeof(BatchItem) == 176, "BatchItem layout");
+static_assert(sizeof(BatchItem) == 192, "BatchItem layout");
 
 // Tile work list of a batch launch: band b owns entries
 // [band_begin[b], band_begin[b] + band_tiles[b]) of `tiles`, each an
@@ -202,8 +205,11 @@ __device__ __forceinline__ uint32_t kth_set_bit(uint64_t m, uint32_t k)
 // node reference of a pooled traversal that has finished
 constexpr uint32_t kDoneRef = 0xffffffffu;
 
+// Four waves per SIMD (128 VGPRs) for every instantiation: left alone, scenes
+// of spheres and meshes take 139 and run at three (the Cornell box, 16 spp:
+// 2.15 ms against 2.01).
 template <uint32_t F, uint32_t W, bool BATCH, bool POOL = false>
-__global__ __launch_bounds__(kBlock) void render_kernel(DevScene sc, KernelParams kp,
+__global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene sc, KernelParams kp,
                                                         const BatchItem *__restrict__ items,
                                                         const BatchTiles *__restrict__ work,
                                                         float4 *__restrict__ acc_buf,
@@ -212,6 +218,7 @@ __global__ __launch_bounds__(kBlock) void render_kernel(DevScene sc, KernelParam
                                                         uint32_t *__restrict__ stage,
                                                         uint32_t *__restrict__ queues)
 {
+    constexpr bool kOrdered = W == 2u;
     extern __shared__ uint32_t lds_stack[];
     uint32_t *stack = lds_stack + threadIdx.x;
     const uint32_t lane = threadIdx.x % 64u;
@@ -234,6 +241,7 @@ __global__ __launch_bounds__(kBlock) void render_kernel(DevScene sc, KernelParam
     uint32_t bounce = 0;
     Traversal tr;
     tr.addr = kLeafRef;  // a lane that is not traversing holds a leaf-flagged reference
+    tr.redo = false;
     uint32_t mode = kWaiting;
     bool need_pixel = true;
     bool blocked = false;  // holds a job whose predecessor has not finished
@@ -398,7 +406,7 @@ __global__ __launch_bounds__(kBlock) void render_kernel(DevScene sc, KernelParam
     for (;;) {
         if constexpr (POOL) {
             static_assert(!(F & kHasMeshes) && W == 2u && !BATCH, "pooled traversal: spheres, BVH2, one image");
-            __shared__ float p_f[7][kBlock];  // inv xyz, ox xyz, t_max of each slot
+            __shared__ float p_f[7][kBlock];  // inv xyz, ox xyz, t_cull of each slot
             __shared__ uint32_t p_addr[kBlock], p_top[kBlock];
             __shared__ uint64_t p_mask[kBlock / 64u];
             __shared__ uint32_t p_alive[kBlock / 64u], p_wait[kBlock / 64u], p_trav[kBlock / 64u];
@@ -415,7 +423,7 @@ __global__ __launch_bounds__(kBlock) void render_kernel(DevScene sc, KernelParam
                 p_f[3][threadIdx.x] = tr.ox.x;
                 p_f[4][threadIdx.x] = tr.ox.y;
                 p_f[5][threadIdx.x] = tr.ox.z;
-                p_f[6][threadIdx.x] = tr.t_max;
+                p_f[6][threadIdx.x] = tr.t_cull;
                 p_addr[threadIdx.x] = tr.addr;
                 p_top[threadIdx.x] = tr.top;
             }
@@ -452,12 +460,12 @@ __global__ __launch_bounds__(kBlock) void render_kernel(DevScene sc, KernelParam
                     slot = ow * 64u + kth_set_bit(p_mask[ow], e - before);
                     wt.inv = mk(p_f[0][slot], p_f[1][slot], p_f[2][slot]);
                     wt.ox = mk(p_f[3][slot], p_f[4][slot], p_f[5][slot]);
-                    wt.t_max = p_f[6][slot];
+                    wt.t_cull = p_f[6][slot];
                     wt.addr = p_addr[slot];
                     wt.top = p_top[slot];
                 }
                 for (uint32_t k = 0; k < node_steps; k++) {
-                    if (!(wt.addr & kLeafRef) && !trav_internal<F, W>(sc, t_min(), ray, lds_stack + slot, kBlock, wt))
+                    if (!(wt.addr & kLeafRef) && !trav_internal<F, W, kOrdered>(sc, t_min(), ray, lds_stack + slot, kBlock, wt))
                         wt.addr = kDoneRef;
                 }
                 if (mine) {
@@ -480,7 +488,7 @@ __global__ __launch_bounds__(kBlock) void render_kernel(DevScene sc, KernelParam
             // of at least `leaf_regroup` lanes. An unflagged tr.addr implies
             // mode == kTraverse: lanes that stop traversing take kLeafRef.
             for (uint32_t k = 0; k < node_steps; k++) {
-                if (!(tr.addr & kLeafRef) && !trav_internal<F, W>(sc, t_min(), ray, stack, kBlock, tr)) {
+                if (!(tr.addr & kLeafRef) && !trav_internal<F, W, kOrdered>(sc, t_min(), ray, stack, kBlock, tr)) {
                     mode = kWaiting;
                     tr.addr = kLeafRef;
                 }
@@ -492,7 +500,7 @@ __global__ __launch_bounds__(kBlock) void render_kernel(DevScene sc, KernelParam
         const uint64_t at_leaf = tracing & ~at_inner;
         if (at_leaf != 0u && (static_cast<uint32_t>(__popcll(at_leaf)) >= leaf_regroup || at_inner == 0u)) {
             if (mode == kTraverse && (tr.addr & kLeafRef) &&
-                !trav_leaf<F, W>(sc, t_min(), ray, stack, kBlock, tr)) {
+                !trav_leaf<F, W, kOrdered>(sc, t_min(), ray, stack, kBlock, tr)) {
                 mode = kWaiting;
                 tr.addr = kLeafRef;
             }
@@ -530,6 +538,8 @@ __global__ __launch_bounds__(kBlock) void render_kernel(DevScene sc, KernelParam
                     begin_job();
                 }
             } else {
+                if (kOrdered && tr.redo)
+                    trav_redo<F>(sc, BATCH ? items[item].root2 : sc.tlas2_root, t_min(), ray, stack, kBlock, tr);
                 bounce++;
                 // each lane's outcome first, then one next_traversal for all
                 // of them (inlined once, so lanes that missed and lanes that
@@ -1367,12 +1377,158 @@ orn_status orn_device_info(orn_ctx *ctx, char *name, size_t name_len, int *compu
 
 namespace {
 
+// The search tree of the ordered traversal (orn_sah.h, orn_trace.h) over the
+// leaves of flagged BVH2 copies: its internal nodes (and a copy of every mesh
+// leaf that enters its BLAS's search tree) are appended to `tlas` and `blas`.
+// Rays get the reference's hits only if its boxes are what its build makes
+// them: finite, each containing the boxes below it, a triangle's own spanning
+// its vertices, every node under one parent. Arrays that are not so keep the
+// reference's order throughout (build returns false and leaves them alone).
+class SearchTree {
+public:
+    std::vector<uint32_t> roots;  // search root reference of each TLAS root
+    uint32_t slots = 1;           // traversal stack entries it needs, in any order of the children
+
+    bool build(const orn_scene_desc *d, const uint32_t *tlas_roots, size_t n_roots, std::vector<orn_bvh_node> &tlas,
+               std::vector<orn_bvh_node> &blas)
+    {
+        if (!nested(d->tlas_nodes, d->tlas_nodes_len) || !nested(d->blas_nodes, d->blas_nodes_len)) return false;
+        std::vector<orn_bvh_node> t = tlas, b = blas;
+        std::vector<uint32_t> blas_root(d->blas_nodes_len, kEmptyRef), blas_slots(d->blas_nodes_len, 0u);
+        std::vector<orn_sah::Leaf> leaves, blas_leaves;
+        std::vector<uint32_t> below(t.size(), 0u);  // stack entries a TLAS leaf's BLAS needs
+        size_t collected = 0;
+        for (size_t i = 0; i < n_roots; i++) {
+            leaves.clear();
+            collect(d->tlas_nodes, tlas_roots[i], leaves);
+            for (orn_sah::Leaf &l : leaves) {
+                const uint32_t idx = l.ref & ~kLeafRef;
+                orn_bvh_node nd = t[idx];
+                std::memcpy(nd.lmin_or_v0, l.box.lo, 12);  // the leaf's own box, in words not otherwise read
+                std::memcpy(nd.lmax_or_v1, l.box.hi, 12);
+                if (nd.node_type != 2u) {
+                    t[idx] = nd;
+                    continue;
+                }
+                const uint32_t r = d->tlas_nodes[idx].left_or_custom_id;
+                if (blas_root[r] == kEmptyRef) {
+                    blas_leaves.clear();
+                    collect(d->blas_nodes, r, blas_leaves);
+                    collected += blas_leaves.size();
+                    if (collected > 2 * d->blas_nodes_len) return false;  // roots inside one another's trees
+                    if (!grow(blas_leaves, b, &blas_root[r])) return false;
+                    blas_slots[r] = pending(b, blas_root[r], nullptr);
+                }
+                nd.left_or_custom_id = blas_root[r];
+                l.ref = kLeafRef | static_cast<uint32_t>(t.size());
+                t.push_back(nd);
+                below.push_back(1u + blas_slots[r]);  // the marker, then the BLAS
+            }
+            uint32_t root = kEmptyRef;
+            if (!grow(leaves, t, &root)) return false;
+            below.resize(t.size(), 0u);
+            roots.push_back(root);
+            slots = std::max(slots, pending(t, root, &below));
+        }
+        if (slots > kMaxStack || t.size() >= kLeafRef || b.size() >= kLeafRef) return false;
+        tlas = std::move(t);
+        blas = std::move(b);
+        return true;
+    }
+
+private:
+    // Levels a search tree may be higher than the balanced one: enough for
+    // the SAH's splits (random spheres and icospheres take 1 or 2), and the
+    // stack it bounds stays close to the reference's.
+    static constexpr uint32_t kExtraHeight = 3;
+
+    static orn_sah::Box box_of(const float *lo, const float *hi)
+    {
+        orn_sah::Box b;
+        std::memcpy(b.lo, lo, 12);
+        std::memcpy(b.hi, hi, 12);
+        return b;
+    }
+
+    static bool nested(const orn_bvh_node *n, size_t len)
+    {
+        std::vector<uint8_t> parents(len, 0);
+        for (size_t i = 0; i < len; i++) {
+            if (n[i].node_type != 0u) continue;
+            const uint32_t kids[2] = {n[i].left_or_custom_id, n[i].right_or_material_index};
+            const orn_sah::Box boxes[2] = {box_of(n[i].lmin_or_v0, n[i].lmax_or_v1),
+                                           box_of(n[i].rmin_or_v2, n[i].rmax_or_v3)};
+            for (int k = 0; k < 2; k++) {
+                const orn_sah::Box &b = boxes[k];
+                const orn_bvh_node &c = n[kids[k]];
+                if (parents[kids[k]]++) return false;
+                for (int a = 0; a < 3; a++) {
+                    if (!std::isfinite(b.lo[a]) || !std::isfinite(b.hi[a]) || !(b.lo[a] <= b.hi[a])) return false;
+                    if (c.node_type == 0u) {
+                        if (!(c.lmin_or_v0[a] >= b.lo[a] && c.rmin_or_v2[a] >= b.lo[a] && c.lmax_or_v1[a] <= b.hi[a] &&
+                              c.rmax_or_v3[a] <= b.hi[a]))
+                            return false;
+                    } else if (c.node_type == 3u) {
+                        const float v0 = c.lmin_or_v0[a], v1 = c.lmax_or_v1[a], v2 = c.rmin_or_v2[a];
+                        if (!(b.lo[a] == std::min(std::min(v0, v1), v2) && b.hi[a] == std::max(std::max(v0, v1), v2)))
+                            return false;
+                    }
+                }
+            }
+        }
+        return true;
+    }
+
+    // The leaves below `root` with the boxes their parents hold for them (a
+    // root that is a leaf has none that is tested: its own words stand in).
+    static void collect(const orn_bvh_node *n, uint32_t root, std::vector<orn_sah::Leaf> &out)
+    {
+        std::vector<uint32_t> todo;
+        auto visit = [&](uint32_t i, const orn_sah::Box &b) {
+            if (n[i].node_type == 0u) todo.push_back(i);
+            else out.push_back({b, kLeafRef | i});
+        };
+        visit(root, box_of(n[root].lmin_or_v0, n[root].lmax_or_v1));
+        while (!todo.empty()) {
+            const orn_bvh_node &nd = n[todo.back()];
+            todo.pop_back();
+            visit(nd.left_or_custom_id, box_of(nd.lmin_or_v0, nd.lmax_or_v1));
+            visit(nd.right_or_material_index, box_of(nd.rmin_or_v2, nd.rmax_or_v3));
+        }
+    }
+
+    static bool grow(std::vector<orn_sah::Leaf> &leaves, std::vector<orn_bvh_node> &nodes, uint32_t *root)
+    {
+        if (leaves.size() == 1) {
+            *root = leaves[0].ref;
+            return true;
+        }
+        const size_t base = nodes.size();
+        if (base + leaves.size() >= kLeafRef) return false;
+        nodes.resize(base + leaves.size() - 1);
+        *root = static_cast<uint32_t>(base);
+        return orn_sah::Builder(leaves, nodes.data() + base, *root)
+            .build(orn_sah::ceil_log2(leaves.size()) + kExtraHeight,
+                   std::min(8u, std::max(1u, std::thread::hardware_concurrency())));
+    }
+
+    // Stack entries a traversal from `ref` on needs whichever child it takes first.
+    static uint32_t pending(const std::vector<orn_bvh_node> &n, uint32_t ref, const std::vector<uint32_t> *below)
+    {
+        if (ref & kLeafRef) return below ? (*below)[ref & ~kLeafRef] : 0u;
+        return 1u + std::max(pending(n, n[ref].left_or_custom_id, below),
+                             pending(n, n[ref].right_or_material_index, below));
+    }
+};
+
 // Uploads validated arrays. `roots` are the TLAS root indices of the scenes
 // the arrays hold (one, or one per image of a batch); their BVH2 and BVH4
-// root references are returned in root2/root4. `slots` is the largest BVH2
+// root references are returned in root2/root4 and their search roots in
+// search_root. `slots` is the largest BVH2
 // stack bound of those scenes.
 orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots, const uint32_t *roots,
-                        size_t n_roots, uint32_t *root2, uint32_t *root4, orn_device_scene **out)
+                        size_t n_roots, uint32_t *root2, uint32_t *root4, uint32_t *search_root,
+                        orn_device_scene **out)
 {
     orn_status st = ORN_OK;
     ORN_TRY(hipSetDevice(ctx->device));
@@ -1447,6 +1603,21 @@ orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots
             }
         for (size_t i = 0; i < n_roots; i++) root2[i] = flag(desc->tlas_nodes, roots[i]);
         ds.tlas2_root = root2[0];
+        SearchTree search;
+        bool ordered = false;
+        try {
+            ordered = search.build(desc, roots, n_roots, t2, b2);
+        } catch (...) {  // no memory for it: the reference's order throughout
+        }
+        for (size_t i = 0; i < n_roots; i++) search_root[i] = ordered ? search.roots[i] : root2[i];
+        ds.search_root = search_root[0];
+        ds.ordered = ordered ? 1u : 0u;
+        s->traversal_slots = ordered ? std::max(slots, search.slots) : slots;
+        float size = 0.0f;  // largest coordinate of the scene
+        for (int a = 0; a < 3; a++)
+            size = std::fmax(size, std::fmax(std::fabs(s->bounds_lo[a]), std::fabs(s->bounds_hi[a])));
+        ds.cull_rel = kCullRel;
+        ds.cull_abs = kCullUlp * size;
         if ((st = upload(s, reinterpret_cast<const float4 *>(t2.data()), 4 * t2.size(), &f4))) return fail(st);
         ds.tlas2 = f4;
         if ((st = upload(s, reinterpret_cast<const float4 *>(b2.data()), 4 * b2.size(), &f4))) return fail(st);
@@ -1525,8 +1696,8 @@ orn_status orn_scene_upload(orn_ctx *ctx, const orn_scene_desc *desc, orn_device
     orn_status st = validate(desc, &slots);
     if (st != ORN_OK) return st;
     const uint32_t root = static_cast<uint32_t>(desc->tlas_nodes_len - 1);
-    uint32_t root2 = 0, root4 = 0;
-    return upload_scene(ctx, desc, slots, &root, 1, &root2, &root4, out);
+    uint32_t root2 = 0, root4 = 0, search_root = 0;
+    return upload_scene(ctx, desc, slots, &root, 1, &root2, &root4, &search_root, out);
 }
 
 orn_status orn_scene_validate(const orn_scene_desc *desc, uint32_t *stack_slots)
@@ -1645,11 +1816,11 @@ hipError_t enqueue_render(orn_device_scene *s, const orn_constant_params *params
     kp.leaf_regroup = tuning.leaf_regroup_lanes;
     kp.node_steps = tuning.node_steps;
     const uint32_t width = tuning.bvh_width == 2u ? 2u : 4u;
-    kp.root = width == 4u ? s->ds.tlas4_root : s->ds.tlas2_root;
+    kp.root = width == 4u ? s->ds.tlas4_root : s->ds.search_root;
     plan_jobs(iterations, params->current_iteration, tuning.samples_per_job,
               uint64_t(kp.tiles_per_xcd) * kTile * kTile, &kp.chunk, &kp.chunks);
     DevScene ds = s->ds;
-    ds.stack_slots = width == 4u ? s->stack_slots4 : s->stack_slots;
+    ds.stack_slots = width == 4u ? s->stack_slots4 : s->traversal_slots;
     const size_t lds = size_t(ds.stack_slots) * kBlock * sizeof(uint32_t);
     kp.epoch = epoch;
     kp.split_pct = tuning.split_percent;
@@ -1888,7 +2059,7 @@ static orn_status trace_rays(orn_device_scene *s, float t_min, const float *rays
     if (e == hipSuccess) e = hipMemcpyAsync(d_rays, rays, n * 6 * sizeof(float), hipMemcpyHostToDevice, st);
     if (e == hipSuccess) {
         DevScene ds = s->ds;
-        ds.stack_slots = s->trace_width == 4u ? s->stack_slots4 : s->stack_slots;
+        ds.stack_slots = s->trace_width == 4u ? s->stack_slots4 : s->traversal_slots;
         const size_t lds = size_t(ds.stack_slots) * kBlock * sizeof(uint32_t);
         const uint32_t blocks = blocks_for(static_cast<uint32_t>(n), kBlock);
         if (packet) {
@@ -2090,7 +2261,7 @@ orn_status merge_scenes(const orn_batch_item *items, size_t n, MergedScene &m, u
 struct orn_batch {
     orn_device_scene *scene;
     size_t n;
-    std::vector<uint32_t> width, height, tiles_x, tiles, px_base, root2, root4, tex_base;
+    std::vector<uint32_t> width, height, tiles_x, tiles, px_base, root2, root4, search_root, tex_base;
     uint32_t total_px;
     uint32_t total_tiles;
     BatchItem *h_items;  // pinned staging of the item table, read by the graph's copy
@@ -2208,7 +2379,7 @@ orn_status capture_batch(orn_batch *b)
     hipStream_t st = s->ctx->stream;
     const uint32_t width = b->tuning.bvh_width == 4u ? 4u : 2u;
     DevScene ds = s->ds;
-    ds.stack_slots = width == 4u ? s->stack_slots4 : s->stack_slots;
+    ds.stack_slots = width == 4u ? s->stack_slots4 : s->traversal_slots;
     const size_t lds = size_t(ds.stack_slots) * kBlock * sizeof(uint32_t);
     KernelParams kp{};
     kp.regroup = b->tuning.regroup_lanes;
@@ -2283,9 +2454,9 @@ orn_status orn_batch_create(orn_ctx *ctx, const orn_batch_item *items, size_t n,
     uint32_t slots = 0;
     orn_status st = merge_scenes(items, n, m, &slots);
     if (st != ORN_OK) return st;
-    std::vector<uint32_t> root2(n), root4(n);
+    std::vector<uint32_t> root2(n), root4(n), search_root(n);
     orn_device_scene *s = nullptr;
-    st = upload_scene(ctx, &m.desc, slots, m.roots.data(), n, root2.data(), root4.data(), &s);
+    st = upload_scene(ctx, &m.desc, slots, m.roots.data(), n, root2.data(), root4.data(), search_root.data(), &s);
     if (st != ORN_OK) return st;
     orn_batch *b = new (std::nothrow) orn_batch();
     if (!b) {
@@ -2296,6 +2467,7 @@ orn_status orn_batch_create(orn_ctx *ctx, const orn_batch_item *items, size_t n,
     b->n = n;
     b->root2 = root2;
     b->root4 = root4;
+    b->search_root = search_root;
     b->tex_base = m.tex_base;
     b->tuning = default_tuning();
     uint32_t base = 0;
@@ -2374,7 +2546,8 @@ orn_status orn_batch_render_async(orn_batch *b, const orn_constant_params *param
         it.iterations = iterations[i];
         it.tiles_x = b->tiles_x[i];
         it.px_base = b->px_base[i];
-        it.root = w4 ? b->root4[i] : b->root2[i];
+        it.root = w4 ? b->root4[i] : b->search_root[i];
+        it.root2 = b->root2[i];
         it.tex_base = b->tex_base[i];
         plan_jobs(iterations[i], params[i].current_iteration, b->tuning.samples_per_job,
                   uint64_t(b->total_tiles) * kTile * kTile, &it.chunk, &it.chunks);

