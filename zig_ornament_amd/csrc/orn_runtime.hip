@@ -8,7 +8,7 @@
 //        pixel and runs all of its samples back to back (the per-pixel RNG
 //        chain is serial, random.wgsl:3-9), regenerating a new camera path as
 //        soon as the previous one ends so that lanes of a wave stay busy
-//        across samples; the framebuffer is post-processed at the end.
+//        across samples; the framebuffer is post-processed by a kernel after it (post_kernel).
 //   bvh_hit (bvh.wgsl:14-137) -> trace_kernel (ray queries).
 //
 // Launch shape: 256-lane workgroups cover 16x16 pixel tiles (a wave is a
@@ -76,7 +76,8 @@ struct BatchItem {
     uint32_t chunks;    // jobs per split pixel
     uint32_t epoch;     // tag of this launch in the stage words
     uint32_t root2;     // TLAS root of the reference's order (rays searched again)
-    uint32_t pad[3];
+    float count;        // State.current_iteration after the render (post_kernel)
+    uint32_t pad[2];
 };
 static_assert(sizeof(BatchItem) == 192, "BatchItem layout");
 
@@ -205,6 +206,26 @@ __device__ __forceinline__ uint32_t kth_set_bit(uint64_t m, uint32_t k)
 // node reference of a pooled traversal that has finished
 constexpr uint32_t kDoneRef = 0xffffffffu;
 
+// The leading kernel arguments as the launch packs them, read again from the
+// kernarg segment where they are used. The camera and the scene's array
+// pointers are needed in shading rounds only; held from the kernel's start
+// they fill the scalar registers and spill into vector lanes, whose reads and
+// writes are vector instructions of the node loop (61-115 spilled scalars,
+// now 2-6). The empty asm hides that every call returns the same address, so
+// no load is moved out of its round. With post_kernel: random spheres 1080p
+// 64 spp 30.4 -> 29.7 ms, instanced icospheres in 2-sample jobs 29.1 -> 26.9,
+// textured, metal and glass icospheres 700x700 8 spp 6.15 -> 4.7.
+struct KernelArgs {
+    DevScene sc;
+    KernelParams kp;
+};
+__device__ __forceinline__ const KernelArgs &reload_args()
+{
+    auto p = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const KernelArgs *)p;
+}
+
 // Four waves per SIMD (128 VGPRs) for every instantiation: left alone, scenes
 // of spheres and meshes take 139 and run at three (the Cornell box, 16 spp:
 // 2.15 ms against 2.01).
@@ -214,7 +235,6 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                                                         const BatchTiles *__restrict__ work,
                                                         float4 *__restrict__ acc_buf,
                                                         uint32_t *__restrict__ rng_buf,
-                                                        float4 *__restrict__ fb,
                                                         uint32_t *__restrict__ stage,
                                                         uint32_t *__restrict__ queues)
 {
@@ -255,7 +275,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
 
     auto params = [&]() -> const orn_constant_params & {
         if constexpr (BATCH) return items[item].p;
-        else return kp.p;
+        else return reload_args().kp.p;
     };
 
     // camera ray of a new sample (camera.wgsl:12-23): 2 jitter draws + 2 lens draws
@@ -278,15 +298,16 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
     };
     // stage word a finished job leaves for its successor
     auto stage_tag = [&](uint32_t jobs_done) {
-        return ((BATCH ? items[item].epoch : kp.epoch) << 16) | jobs_done;
+        return ((BATCH ? items[item].epoch : reload_args().kp.epoch) << 16) | jobs_done;
     };
     auto job_ready = [&]() { return job == 0u || load_coherent(stage + pix) == stage_tag(job); };
-    // End of a job: the state goes back to memory; the last job of a pixel
-    // also writes the framebuffer (pathtracer.wgsl:81-93), the others
-    // release the pixel to its next job.
+    // End of a job: the state goes back to memory (post_kernel reads the
+    // accumulation once the launch is done); every job but a pixel's last
+    // releases the pixel to the next one.
     auto end_job = [&]() {
-        if (kp.cost)  // the pixel's cost for the next render's queue order
-            __hip_atomic_fetch_add(kp.cost + pix, device_ticks() - job_t0, __ATOMIC_RELAXED,
+        uint32_t *cost = reload_args().kp.cost;
+        if (cost)  // the pixel's cost for the next render's queue order
+            __hip_atomic_fetch_add(cost + pix, device_ticks() - job_t0, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
         if (job + 1u < lane_chunks) {  // handed on; released at the wave's next flush
             store_coherent(acc_rsrc, pix, acc);
@@ -301,18 +322,6 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
         }
         acc_buf[pix] = acc;  // the pixel's last job: read next by a later launch
         rng_buf[pix] = rng;
-        const orn_constant_params &p = params();
-        float4 o;
-        o.x = fminf(fmaxf(acc.x / cur, 0.0f), 1.0f);
-        o.y = fminf(fmaxf(acc.y / cur, 0.0f), 1.0f);
-        o.z = fminf(fmaxf(acc.z / cur, 0.0f), 1.0f);
-        o.w = fminf(fmaxf(acc.w / cur, 0.0f), 1.0f);
-        o.x = pow_f(o.x, p.inverted_gamma);
-        o.y = pow_f(o.y, p.inverted_gamma);
-        o.z = pow_f(o.z, p.inverted_gamma);
-        const uint32_t row = p.flip_y < 1u ? y : p.height - y - 1u;
-        const uint32_t base = BATCH ? items[item].px_base : 0u;
-        fb[base + row * p.width + x] = o;
     };
     // Accumulate finished samples, finish samples that need no traversal
     // (depth exhausted), and set up the next traversal; a finished job asks
@@ -353,7 +362,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
     // per-sample increments reach.
     auto begin_job = [&]() {
         const orn_constant_params &p = params();
-        if (kp.cost) job_t0 = device_ticks();
+        if (reload_args().kp.cost) job_t0 = device_ticks();
         if (job == 0u) {  // state left by an earlier launch
             rng = rng_buf[pix];
             acc = acc_buf[pix];
@@ -364,9 +373,9 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
             rng = load_coherent(rng_buf + pix);
             acc = load_coherent(acc_rsrc, pix);
         }
-        const uint32_t iters = BATCH ? items[item].iterations : kp.iterations;
+        const uint32_t iters = BATCH ? items[item].iterations : reload_args().kp.iterations;
         const uint32_t spp = iters > 1u ? iters : 1u;
-        const uint32_t chunk = lane_chunks == 1u ? spp : (BATCH ? items[item].chunk : kp.chunk);
+        const uint32_t chunk = lane_chunks == 1u ? spp : (BATCH ? items[item].chunk : reload_args().kp.chunk);
         const uint32_t first = job * chunk;
         cur = first == 0u ? p.current_iteration : p.current_iteration + static_cast<float>(first);
         left = min(chunk, spp - first);
@@ -386,19 +395,23 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
         }
     };
     // jobs per band: band_px - split whole pixels, then split x max_chunks
-    const uint32_t max_chunks = BATCH ? work->max_chunks : kp.chunks;
-    const uint32_t split_pct = kp.split_pct;
     auto band_pixels = [&](uint32_t b) -> uint32_t {
         if constexpr (BATCH) return work->band_tiles[b] * (kTile * kTile);
-        const uint32_t first = b * kp.tiles_per_xcd;
-        return first >= kp.tiles ? 0u : min(kp.tiles_per_xcd, kp.tiles - first) * (kTile * kTile);
+        const KernelParams &k = reload_args().kp;
+        const uint32_t first = b * k.tiles_per_xcd;
+        return first >= k.tiles ? 0u : min(k.tiles_per_xcd, k.tiles - first) * (kTile * kTile);
     };
+    auto split_pixels = [&](uint32_t px) {
+        const uint32_t pct = reload_args().kp.split_pct;
+        return px / 100u * pct + px % 100u * pct / 100u;
+    };
+    auto max_chunks = [&]() { return BATCH ? work->max_chunks : reload_args().kp.chunks; };
 
     uint32_t band = blockIdx.x % kXcds;  // wave-uniform
     uint32_t bands_left = kXcds - 1u;    // bands to visit after this one
     uint32_t band_px = band_pixels(band);
-    uint32_t band_split = band_px / 100u * split_pct + band_px % 100u * split_pct / 100u;
-    uint32_t band_jobs = band_px - band_split + band_split * max_chunks;
+    uint32_t band_split = split_pixels(band_px);
+    uint32_t band_jobs = band_px - band_split + band_split * max_chunks();
     const uint32_t regroup = kp.regroup;
     const uint32_t leaf_regroup = kp.leaf_regroup;
     const uint32_t node_steps = kp.node_steps;
@@ -557,7 +570,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                     f3 w;
                     const uint32_t tex_count = params().textures_count;
                     const uint32_t tex_base = BATCH ? items[item].tex_base : 0u;
-                    done = !shade<F>(sc, tex_count, tex_base, ray, tr.h, rng, next, w);
+                    done = !shade<F>(reload_args().sc, tex_count, tex_base, ray, tr.h, rng, next, w);
                     if (done) {
                         color = thr * w;
                     } else {
@@ -586,6 +599,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                 if (q >= band_jobs) {
                     if (bands_left == 0u) mode = kDone;  // every band has run out
                 } else {
+                    const KernelParams &k = reload_args().kp;
                     // whole pixel, or job c of split pixel qp
                     const uint32_t bulk = band_px - band_split;
                     uint32_t c = 0, qp = q;
@@ -595,7 +609,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                     }
                     // position qp of the band's queue -> tile-pixel of the band
                     const uint32_t qpx =
-                        kp.order ? kp.order[(BATCH ? work->band_begin[band] : band * kp.tiles_per_xcd) *
+                        k.order ? k.order[(BATCH ? work->band_begin[band] : band * k.tiles_per_xcd) *
                                                 (kTile * kTile) + qp]
                                  : qp;
                     const uint32_t within = qpx % (kTile * kTile);
@@ -609,11 +623,11 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                         h = items[item].p.height;
                         chunks = items[item].chunks;
                     } else {
-                        tile = band * kp.tiles_per_xcd + qpx / (kTile * kTile);
-                        tiles_x = kp.tiles_x;
-                        w = kp.p.width;
-                        h = kp.p.height;
-                        chunks = kp.chunks;
+                        tile = band * k.tiles_per_xcd + qpx / (kTile * kTile);
+                        tiles_x = k.tiles_x;
+                        w = k.p.width;
+                        h = k.p.height;
+                        chunks = k.chunks;
                     }
                     x = (tile % tiles_x) * kTile + within % kTile;
                     y = (tile / tiles_x) * kTile + within / kTile;
@@ -642,12 +656,53 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                 band = band + 1u == kXcds ? 0u : band + 1u;
                 bands_left--;
                 band_px = band_pixels(band);
-                band_split = band_px / 100u * split_pct + band_px % 100u * split_pct / 100u;
-                band_jobs = band_px - band_split + band_split * max_chunks;
+                band_split = split_pixels(band_px);
+                band_jobs = band_px - band_split + band_split * max_chunks();
             }
         }
     }
     flush_releases();  // no successor may wait on a release this wave holds
+}
+
+// main_post_processing (pathtracer.wgsl:81-93) of a finished render: the mean
+// over `count` samples, clamped, gamma-corrected, into the framebuffer. Its
+// own launch, one lane per pixel, bound by its 32 bytes per pixel: written by
+// render_kernel as each pixel's last sample ended, the three powers ran for
+// one or two lanes of a wave at a time, ~400 vector instructions of each such
+// shading round.
+__device__ __forceinline__ void post_pixel(const orn_constant_params &p, float count, uint32_t x, uint32_t y,
+                                           const float4 *__restrict__ acc, float4 *__restrict__ fb)
+{
+    const float4 a = acc[y * p.width + x];
+    float4 o;
+    o.x = fminf(fmaxf(a.x / count, 0.0f), 1.0f);
+    o.y = fminf(fmaxf(a.y / count, 0.0f), 1.0f);
+    o.z = fminf(fmaxf(a.z / count, 0.0f), 1.0f);
+    o.w = fminf(fmaxf(a.w / count, 0.0f), 1.0f);
+    o.x = pow_f(o.x, p.inverted_gamma);
+    o.y = pow_f(o.y, p.inverted_gamma);
+    o.z = pow_f(o.z, p.inverted_gamma);
+    const uint32_t row = p.flip_y < 1u ? y : p.height - y - 1u;
+    fb[row * p.width + x] = o;
+}
+
+__global__ __launch_bounds__(kBlock) void post_kernel(orn_constant_params p, float count,
+                                                      const float4 *__restrict__ acc, float4 *__restrict__ fb)
+{
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i < p.width * p.height) post_pixel(p, count, i % p.width, i / p.width, acc, fb);
+}
+
+// Every image of a batch: a workgroup per entry of the tile work list.
+__global__ __launch_bounds__(kBlock) void post_batch_kernel(const BatchItem *__restrict__ items,
+                                                            const BatchTiles *__restrict__ work,
+                                                            const float4 *__restrict__ acc, float4 *__restrict__ fb)
+{
+    const uint2 e = work->tiles[blockIdx.x];
+    const BatchItem &it = items[e.x];
+    const uint32_t x = (e.y % it.tiles_x) * kTile + threadIdx.x % kTile;
+    const uint32_t y = (e.y / it.tiles_x) * kTile + threadIdx.x / kTile;
+    if (x < it.p.width && y < it.p.height) post_pixel(it.p, it.count, x, y, acc + it.px_base, fb + it.px_base);
 }
 
 __global__ void reset_queues_kernel(uint32_t *q)
@@ -1168,6 +1223,21 @@ bool splits_exactly(float current_iteration, uint32_t iterations)
            double(current_iteration) + spp <= 16777216.0;
 }
 
+// State.current_iteration after a render: 1 added per sample in f32, which
+// stops changing the counter once it is large.
+float count_after(float current_iteration, uint32_t iterations)
+{
+    const uint32_t spp = iterations > 1u ? iterations : 1u;
+    if (splits_exactly(current_iteration, iterations)) return current_iteration + static_cast<float>(spp);
+    float c = current_iteration;
+    for (uint32_t i = 0; i < spp; i++) {
+        const float next = c + 1.0f;
+        if (!(next != c)) break;
+        c = next;
+    }
+    return c;
+}
+
 void plan_jobs(uint32_t iterations, float current_iteration, uint32_t samples_per_job, uint64_t band_pixels,
                uint32_t *chunk, uint32_t *chunks)
 {
@@ -1192,7 +1262,6 @@ struct LaunchArgs {
     const BatchTiles *work;
     float4 *acc;
     uint32_t *rng;
-    float4 *fb;
     uint32_t *stage;
     uint32_t *queues;
     uint32_t total_tiles;
@@ -1220,7 +1289,7 @@ hipError_t launch_render_k(uint32_t per_cu, uint32_t cus, size_t lds, hipStream_
     grid = std::min(grid, blocks_for(a.total_tiles, kXcds) * kXcds);
     grid = std::max(kXcds, grid / kXcds * kXcds);
     render_kernel<F, W, BATCH, POOL>
-        <<<grid, kBlock, lds, st>>>(ds, a.kp, a.items, a.work, a.acc, a.rng, a.fb, a.stage, a.queues);
+        <<<grid, kBlock, lds, st>>>(ds, a.kp, a.items, a.work, a.acc, a.rng, a.stage, a.queues);
     return hipGetLastError();
 }
 
@@ -1798,7 +1867,8 @@ orn_status orn_target_destroy(orn_target *t)
 namespace {
 
 // The render launch of one image on buffers the caller provides: the
-// queues are reset and the kernel enqueued on `st`. `epoch` tags this
+// queues are reset and the kernel enqueued on `st`, then, with a framebuffer,
+// its post-processing. `epoch` tags this
 // launch's stage words (unique among the launches that used `stage` since it
 // was last cleared). Allocates nothing.
 hipError_t enqueue_render(orn_device_scene *s, const orn_constant_params *params, uint32_t iterations,
@@ -1827,10 +1897,14 @@ hipError_t enqueue_render(orn_device_scene *s, const orn_constant_params *params
     kp.pixels = params->width * params->height;
     kp.order = order;
     kp.cost = cost;
-    LaunchArgs a{kp, nullptr, nullptr, acc, rng, fb, stage, queues, kp.tiles, tuning.workgroup_pool != 0u};
+    LaunchArgs a{kp, nullptr, nullptr, acc, rng, stage, queues, kp.tiles, tuning.workgroup_pool != 0u};
     reset_queues_kernel<<<1, 64, 0, st>>>(queues);
-    return launch_render<false>(s->features, width, tuning.workgroups_per_cu,
-                                static_cast<uint32_t>(s->ctx->compute_units), lds, st, ds, a);
+    const hipError_t e = launch_render<false>(s->features, width, tuning.workgroups_per_cu,
+                                              static_cast<uint32_t>(s->ctx->compute_units), lds, st, ds, a);
+    if (e != hipSuccess || !fb) return e;
+    post_kernel<<<blocks_for(kp.pixels, kBlock), kBlock, 0, st>>>(
+        *params, count_after(params->current_iteration, iterations), acc, fb);
+    return hipGetLastError();
 }
 
 // Buffers of a target's cost-ordered queues, allocated on first use; the
@@ -1904,7 +1978,7 @@ orn_status orn_render_async(orn_target *t, const orn_constant_params *params, ui
         // continues it (a render of k then n - k samples from
         // current_iteration + k gives the same bits as one of n).
         const uint32_t first = std::max(1u, iterations / 8u);
-        ORN_TRY(enqueue_render(s, params, first, t->tuning, t->acc, t->rng, t->fb, t->stage, t->queues, t->epoch,
+        ORN_TRY(enqueue_render(s, params, first, t->tuning, t->acc, t->rng, nullptr, t->stage, t->queues, t->epoch,
                                st, nullptr, t->cost));
         next_epoch();
         enqueue_queue_order(t, st);
@@ -2365,7 +2439,7 @@ hipError_t ensure_batch_cost_order(orn_batch *b, hipStream_t st)
     return hipGetLastError();
 }
 
-// Captures [item table copy, queue reset, render launch] as one graph; with
+// Captures [item table copy, queue reset, render launch, post-processing] as one graph; with
 // tuning cost_order, the queue-order kernels run between the copy and the
 // launch, on the costs the previous replay recorded.
 orn_status capture_batch(orn_batch *b)
@@ -2393,7 +2467,7 @@ orn_status capture_batch(orn_batch *b)
         kp.order = b->order;
         kp.cost = b->cost;
     }
-    LaunchArgs a{kp, b->d_items, b->d_work, b->acc, b->rng, b->fb, b->stage, b->queues, b->total_tiles};
+    LaunchArgs a{kp, b->d_items, b->d_work, b->acc, b->rng, b->stage, b->queues, b->total_tiles};
     ORN_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
     hipError_t e = hipMemcpyAsync(b->d_items, b->h_items, b->n * sizeof(BatchItem), hipMemcpyHostToDevice, st);
     if (e == hipSuccess && by_cost) {
@@ -2410,6 +2484,10 @@ orn_status capture_batch(orn_batch *b)
     if (e == hipSuccess)
         e = launch_render<true>(s->features, width, b->tuning.workgroups_per_cu,
                                 static_cast<uint32_t>(s->ctx->compute_units), lds, st, ds, a);
+    if (e == hipSuccess) {
+        post_batch_kernel<<<b->total_tiles, kBlock, 0, st>>>(b->d_items, b->d_work, b->acc, b->fb);
+        e = hipGetLastError();
+    }
     hipGraph_t g = nullptr;
     const hipError_t e2 = hipStreamEndCapture(st, &g);
     if (e == hipSuccess) e = e2;
@@ -2548,6 +2626,7 @@ orn_status orn_batch_render_async(orn_batch *b, const orn_constant_params *param
         it.px_base = b->px_base[i];
         it.root = w4 ? b->root4[i] : b->search_root[i];
         it.root2 = b->root2[i];
+        it.count = count_after(params[i].current_iteration, iterations[i]);
         it.tex_base = b->tex_base[i];
         plan_jobs(iterations[i], params[i].current_iteration, b->tuning.samples_per_job,
                   uint64_t(b->total_tiles) * kTile * kTile, &it.chunk, &it.chunks);
