@@ -963,7 +963,7 @@ __device__ __forceinline__ f3 continue_path(const DevScene &sc, const orn_consta
         if (!bvh_hit<F, 2, kNodeSteps>(sc, p.ray_cast_epsilon, ray, stack, kBlock, h)) return thr * sky(ray.d);
         Ray next;
         f3 w;
-        if (shade<F>(sc, p.textures_count, 0u, ray, h, rng, next, w)) {
+        if (shade<F>(sc, p.textures_count, 0u, ray, normalize(ray.d), h, rng, next, w)) {
             ray = next;
             thr = thr * w;
         } else {

@@ -559,8 +559,8 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                 // scattered share its code)
                 bool done;
                 f3 color;
+                const f3 ud = normalize(ray.d);
                 if (!tr.hit) {
-                    const f3 ud = normalize(ray.d);
                     const float tt = 0.5f * (ud.y + 1.0f);
                     const float a = (1.0f - tt) * 1.0f;
                     done = true;
@@ -570,7 +570,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                     f3 w;
                     const uint32_t tex_count = params().textures_count;
                     const uint32_t tex_base = BATCH ? items[item].tex_base : 0u;
-                    done = !shade<F>(reload_args().sc, tex_count, tex_base, ray, tr.h, rng, next, w);
+                    done = !shade<F>(reload_args().sc, tex_count, tex_base, ray, ud, tr.h, rng, next, w);
                     if (done) {
                         color = thr * w;
                     } else {

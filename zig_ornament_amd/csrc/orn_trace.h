@@ -804,9 +804,11 @@ __device__ __forceinline__ Surface surface(const DevScene &sc, uint32_t textures
 // into the shared table, and 0xffffffff for "none"). Textures beyond what was
 // uploaded read as "no texture" (the reference would index its binding array
 // out of range there).
+// `ud` is normalize(ray.d), computed by the caller once for every kind of lane
+// (sky, metal and dielectric lanes of a wave would each run their own).
 template <uint32_t F>
 __device__ __forceinline__ bool shade(const DevScene &sc, uint32_t textures_count, uint32_t tex_base,
-                                      const Ray &ray, const Hit &h, uint32_t &rng, Ray &next, f3 &weight)
+                                      const Ray &ray, f3 ud, const Hit &h, uint32_t &rng, Ray &next, f3 &weight)
 {
     const f3 p = ray.o + h.t * ray.d;
     const Material m = load_material(sc, h.material);
@@ -864,11 +866,11 @@ __device__ __forceinline__ bool shade(const DevScene &sc, uint32_t textures_coun
         f3 dir;
         bool cont;
         if (m.type == 0u) {
-            dir = normal + normalize(s);
+            dir = normal + normalize_draw(s);
             if (near_zero(dir)) dir = normal;
             cont = true;
         } else {
-            dir = reflect_dir(normalize(ray.d), normal) + m.fuzz * s;
+            dir = reflect_dir(ud, normal) + m.fuzz * s;
             cont = dot(dir, normal) > 0.0f;  // absorbed below the surface
         }
         next.o = p;
@@ -883,15 +885,14 @@ __device__ __forceinline__ bool shade(const DevScene &sc, uint32_t textures_coun
     switch (m.type) {
     case 2u: {  // material.wgsl:36-59
         const float ratio = front ? (1.0f / m.ior) : m.ior;
-        const f3 ud = normalize(ray.d);
         const float cos_theta = fminf(dot(-ud, normal), 1.0f);
-        const float sin_theta = sqrtf(1.0f - cos_theta * cos_theta);
+        const float sin_theta = sqrt_tame(1.0f - cos_theta * cos_theta);
         const bool cannot_refract = ratio * sin_theta > 1.0f;
         bool reflect = cannot_refract;
         if (!reflect) {  // the draw happens only when refraction is possible
             float r0 = (1.0f - ratio) / (1.0f + ratio);
             r0 = r0 * r0;
-            const float refl = r0 + (1.0f - r0) * pow_f(1.0f - cos_theta, 5.0f);
+            const float refl = r0 + (1.0f - r0) * pow_draw(1.0f - cos_theta, 5.0f);
             reflect = refl > rng_f32(rng);
         }
         next.o = p;
@@ -928,7 +929,7 @@ __device__ __forceinline__ bool scatter(const DevScene &sc, const Surface &srf, 
         f3 dir;
         bool cont;
         if (m.type == 0u) {
-            dir = normal + normalize(s);
+            dir = normal + normalize_draw(s);
             if (near_zero(dir)) dir = normal;
             cont = true;
         } else {
@@ -949,13 +950,13 @@ __device__ __forceinline__ bool scatter(const DevScene &sc, const Surface &srf, 
         const float ratio = front ? (1.0f / m.ior) : m.ior;
         const f3 ud = normalize(ray.d);
         const float cos_theta = fminf(dot(-ud, normal), 1.0f);
-        const float sin_theta = sqrtf(1.0f - cos_theta * cos_theta);
+        const float sin_theta = sqrt_tame(1.0f - cos_theta * cos_theta);
         const bool cannot_refract = ratio * sin_theta > 1.0f;
         bool reflect = cannot_refract;
         if (!reflect) {  // the draw happens only when refraction is possible
             float r0 = (1.0f - ratio) / (1.0f + ratio);
             r0 = r0 * r0;
-            const float refl = r0 + (1.0f - r0) * pow_f(1.0f - cos_theta, 5.0f);
+            const float refl = r0 + (1.0f - r0) * pow_draw(1.0f - cos_theta, 5.0f);
             reflect = refl > rng_f32(rng);
         }
         next.o = p;
