@@ -125,3 +125,18 @@ def test_boxes_that_are_not_nested_keep_the_references_order(device, change):
         arrays.tlas_nodes["rmax_or_v3"][inner[::4]] += np.float32(-0.3 if change == "shrunk" else np.inf)
     print(f"[search] {change}: {len(rays)} rays", flush=True)
     assert _compare(device, arrays, arrays, rays, 0.001) > 0.05
+
+
+def test_spheres_with_any_transform_keep_the_whole_matrix(device):
+    """One sheared, rotated or mirrored sphere among them sends every sphere
+    leaf through its whole matrix."""
+    spec = _spec("sheared", _grid(3))
+    arrays = zo.Bvh(W.build_scene(spec))
+    rays = _rays(spec, arrays, seed=9)
+    plain = _compare(device, arrays, arrays, rays, 0.001)
+    arrays = copy.copy(arrays)
+    arrays.transforms[8, 4] += np.float32(0.25)  # off the diagonal of a leaf's inverse
+    arrays.transforms[10, 0] *= np.float32(-1.0)
+    print(f"[search] sheared: {len(rays)} rays", flush=True)
+    assert plain > 0.05 and _compare(device, arrays, arrays, rays, 0.001) > 0.05
+    assert _compare(device, arrays, arrays, rays, 0.0) > 0.05

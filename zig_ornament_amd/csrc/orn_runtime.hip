@@ -1446,6 +1446,38 @@ orn_status orn_device_info(orn_ctx *ctx, char *name, size_t name_len, int *compu
 
 namespace {
 
+// Whether every sphere leaf of the TLAS is scaled along the axes and moved
+// (sphere_leaf, sphere_centre in orn_trace.h).
+bool spheres_are_plain(const orn_scene_desc *d)
+{
+    for (size_t i = 0; i < d->tlas_nodes_len; i++) {
+        if (d->tlas_nodes[i].node_type != 1u) continue;
+        const float *inv = d->transforms + 32 * size_t(d->tlas_nodes[i].transform_id), *m = inv + 16;
+        for (int c = 0; c < 4; c++)
+            for (int r = 0; r < 3; r++) {
+                const float a = inv[4 * c + r], b = m[4 * c + r];
+                if (!std::isfinite(a) || !std::isfinite(b)) return false;
+                if (c < 3 && c != r && a != 0.0f) return false;
+                if (c == 3 && b == 0.0f && std::signbit(b)) return false;
+            }
+    }
+    return true;
+}
+
+// Puts the diagonal and the translation of plain spheres' inverse transforms
+// into words of their leaves that nothing else reads.
+void fill_sphere_leaves(const orn_scene_desc *d, std::vector<orn_bvh_node> &nodes)
+{
+    for (orn_bvh_node &nd : nodes) {
+        if (nd.node_type != 1u) continue;
+        const float *inv = d->transforms + 32 * size_t(nd.transform_id);
+        for (int a = 0; a < 3; a++) {
+            nd.rmin_or_v2[a] = inv[5 * a];
+            nd.rmax_or_v3[a] = inv[12 + a];
+        }
+    }
+}
+
 // The search tree of the ordered traversal (orn_sah.h, orn_trace.h) over the
 // leaves of flagged BVH2 copies: its internal nodes (and a copy of every mesh
 // leaf that enters its BLAS's search tree) are appended to `tlas` and `blas`.
@@ -1672,6 +1704,8 @@ orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots
             }
         for (size_t i = 0; i < n_roots; i++) root2[i] = flag(desc->tlas_nodes, roots[i]);
         ds.tlas2_root = root2[0];
+        ds.plain_spheres = spheres_are_plain(desc) ? 1u : 0u;
+        if (ds.plain_spheres) fill_sphere_leaves(desc, t2);
         SearchTree search;
         bool ordered = false;
         try {
@@ -1706,6 +1740,7 @@ orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots
                 blas_ref[r] = b4.build(r);
                 nd.left_or_custom_id = blas_ref[r];
             }
+        if (ds.plain_spheres) fill_sphere_leaves(desc, leaves);
         std::vector<uint32_t> memo(desc->blas_nodes_len, 0xffffffffu);
         uint32_t slots4 = 1;
         for (size_t i = 0; i < n_roots; i++)
