@@ -47,6 +47,15 @@ constexpr uint32_t kXcds = 8;
 // 2000x1000, 15 spp: 12.2 ms, now 7.5; instanced icospheres in 2-sample jobs
 // 26.6 ms, now 24.2; random spheres 64 spp 25.8, now 25.2).
 constexpr uint32_t kQueueStride = 32;
+// A draw takes more jobs than the wave's lanes ask for, for its next ones: a
+// kAheadShare-th of what an even share of the band's remaining jobs is per
+// wave, so that the reserves shrink to nothing towards the band's end. Fewer
+// draws queue up at a counter (2000x1000, 15 spp: 7.5 -> 7.1 ms; instanced
+// icospheres 22.8 -> 22.4); larger shares leave jobs with busy waves at the
+// end (a quarter instead of a 64th: a 16-image batch 12.4 -> 15 ms). Only for
+// whole pixels: a wave must not hold a split pixel's job back while all its
+// lanes wait for jobs that other waves hold back.
+constexpr uint32_t kAheadShare = 64, kAheadMost = 64;
 constexpr uint32_t kQueueWords = kXcds * kQueueStride;
 constexpr uint32_t kMaxStack = 63;  // the reference's private stack has 64 slots
 constexpr uint64_t kMaxPixels = 1ull << 28;  // per target or batch: 4 GiB of accumulation
@@ -416,6 +425,9 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
 
     uint32_t band = blockIdx.x % kXcds;  // wave-uniform
     uint32_t bands_left = kXcds - 1u;    // bands to visit after this one
+    // Jobs [held_at, held_at + held) of the band are the wave's, drawn but not
+    // yet given to lanes; its next draw takes `ahead` more than lanes ask for.
+    uint32_t held_at = 0, held = 0, ahead = 0;
     uint32_t band_px = band_pixels(band);
     uint32_t band_split = split_pixels(band_px);
     uint32_t band_jobs = band_px - band_split + band_split * max_chunks();
@@ -598,11 +610,21 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
             if (needy == 0u) break;
             const int leader = __ffsll(static_cast<unsigned long long>(needy)) - 1;
             const uint32_t count = static_cast<uint32_t>(__popcll(needy));
-            uint32_t base = 0;
-            if (lane == static_cast<uint32_t>(leader)) base = atomicAdd(queues + band * kQueueStride, count);
-            base = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(base), leader));
-            if (mode == kWaiting && need_pixel) {
-                const uint32_t q = base + static_cast<uint32_t>(__popcll(needy & ((1ull << lane) - 1ull)));
+            if (held == 0u) {
+                held = count + ahead;
+                uint32_t base = 0;
+                if (lane == static_cast<uint32_t>(leader)) base = atomicAdd(queues + band * kQueueStride, held);
+                held_at = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(base), leader));
+                const bool whole = reload_args().kp.split_pct == 0u || max_chunks() == 1u;
+                ahead = whole && held_at < band_jobs ? min((band_jobs - held_at) / (gridDim.x / 2u * kAheadShare), kAheadMost)
+                                                     : 0u;
+            }
+            const uint32_t rank = static_cast<uint32_t>(__popcll(needy & ((1ull << lane) - 1ull)));
+            const uint32_t q = held_at + rank;
+            const uint32_t taken = min(count, held);
+            held -= taken;
+            held_at += taken;
+            if (mode == kWaiting && need_pixel && rank < taken) {
                 if (q >= band_jobs) {
                     if (bands_left == 0u) mode = kDone;  // every band has run out
                 } else {
@@ -659,7 +681,9 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                     }
                 }
             }
-            if (base + count > band_jobs && bands_left != 0u) {  // the band ran out (wave-uniform)
+            if (held_at >= band_jobs) held = 0u;  // what is left of it lies past the band's end
+            if (held_at >= band_jobs && bands_left != 0u) {  // the band ran out (wave-uniform)
+                ahead = 0u;
                 band = band + 1u == kXcds ? 0u : band + 1u;
                 bands_left--;
                 band_px = band_pixels(band);
