@@ -1696,10 +1696,6 @@ orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots
         return e;
     };
     const float4 *f4 = nullptr;
-    if ((st = upload(s, reinterpret_cast<const float4 *>(desc->tlas_nodes), 4 * desc->tlas_nodes_len, &f4))) return fail(st);
-    ds.tlas = f4;
-    if ((st = upload(s, reinterpret_cast<const float4 *>(desc->blas_nodes), 4 * desc->blas_nodes_len, &f4))) return fail(st);
-    ds.blas = f4;
     if ((st = upload(s, reinterpret_cast<const float4 *>(desc->normals), desc->normals_len, &f4))) return fail(st);
     ds.normals = f4;
     if ((st = upload(s, reinterpret_cast<const float4 *>(desc->transforms), 4 * desc->transforms_len, &f4))) return fail(st);
@@ -1752,10 +1748,21 @@ orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots
             size = std::fmax(size, std::fmax(std::fabs(s->bounds_lo[a]), std::fabs(s->bounds_hi[a])));
         ds.cull_rel = kCullRel;
         ds.cull_abs = kCullUlp * size;
+        // one array: the BLAS nodes behind the TLAS's
+        const size_t tlas_n = t2.size();
+        if (tlas_n + b2.size() >= kLeafRef) return fail(ORN_ERROR_OUT_OF_MEMORY);
+        const uint32_t shift = static_cast<uint32_t>(tlas_n);  // leaves the flag alone
+        for (orn_bvh_node &nd : t2)
+            if (nd.node_type == 2u) nd.left_or_custom_id += shift;
+        for (orn_bvh_node &nd : b2)
+            if (nd.node_type == 0u) {
+                nd.left_or_custom_id += shift;
+                nd.right_or_material_index += shift;
+            }
+        t2.insert(t2.end(), b2.begin(), b2.end());
         if ((st = upload(s, reinterpret_cast<const float4 *>(t2.data()), 4 * t2.size(), &f4))) return fail(st);
-        ds.tlas2 = f4;
-        if ((st = upload(s, reinterpret_cast<const float4 *>(b2.data()), 4 * b2.size(), &f4))) return fail(st);
-        ds.blas2 = f4;
+        ds.nodes2 = f4;
+        ds.blas2 = f4 + 4 * tlas_n;
     }
     // derived BVH4 arrays and the TLAS copy whose mesh leaves point at
     // their BLAS's BVH4 root
