@@ -483,7 +483,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                 Traversal wt;
                 wt.addr = kDoneRef;
                 wt.top = 0;
-                wt.in_tlas = true;
+                wt.blas_top = kInTlas;
                 wt.hit = false;
                 if (mine) {
                     const uint32_t p1 = n0, p2 = n0 + n1, p3 = n0 + n1 + n2;

@@ -15,6 +15,7 @@
 namespace orn {
 
 constexpr uint32_t kFinishedTraverseBlas = 0xffffffffu;  // pathtracer.wgsl:19
+constexpr uint32_t kInTlas = 0xffffffffu;
 constexpr float kTMaxInit = 3.40282e+38f;                 // bvh.wgsl:23
 // slack of the ordered search's distance cull (trav_cull)
 constexpr float kCullRel = 1.0f / 512.0f;    // of t
@@ -275,7 +276,7 @@ struct Traversal {
     uint32_t addr;  // next node to visit
     uint32_t top;   // pending entries in the LDS column
     uint32_t material_index, inv_tid;  // of the mesh being traversed
-    bool in_tlas;
+    uint32_t blas_top;  // `top` when the ray entered the BLAS it is in (kInTlas: none)
     bool hit;
     bool early;  // ORD: the closest hit lies in front of its own box
     bool redo;   // ORD: the closest hit needs the reference's order (see above)
@@ -299,7 +300,7 @@ __device__ __forceinline__ void trav_begin(uint32_t root, const Ray &world, Trav
     tr.top = 0u;
     tr.material_index = 0u;
     tr.inv_tid = 0u;
-    tr.in_tlas = true;
+    tr.blas_top = kInTlas;
     tr.hit = false;
 }
 
@@ -312,21 +313,20 @@ __device__ __forceinline__ void pin_node(float4 &a, float4 &b, float4 &c, float4
 }
 
 // Takes the next pending node off the lane's stack; false when none is left.
+// A BLAS is done when the stack is down to where it was on entering it (the
+// reference pushes a marker instead, bvh.wgsl:88-95).
 template <uint32_t F>
-__device__ __forceinline__ bool trav_pop(const DevScene &sc, const Ray &world, uint32_t *stack,
-                                         uint32_t stride, Traversal &tr)
+__device__ __forceinline__ bool trav_pop(uint32_t *stack, uint32_t stride, Traversal &tr)
 {
     if (tr.top == 0u) return false;
-    tr.addr = stack[(--tr.top) * stride];
-    if ((F & kHasMeshes) && tr.addr == kFinishedTraverseBlas) {
+    if ((F & kHasMeshes) && tr.top == tr.blas_top) {
         // back in the TLAS: the world-space ray's reciprocal, kept from
         // trav_begin
-        tr.in_tlas = true;
+        tr.blas_top = kInTlas;
         tr.inv = tr.winv;
         tr.ox = tr.wox;
-        if (tr.top == 0u) return false;
-        tr.addr = stack[(--tr.top) * stride];
     }
+    tr.addr = stack[(--tr.top) * stride];
     return true;
 }
 
@@ -403,10 +403,10 @@ __device__ __forceinline__ bool trav_internal(const DevScene &sc, float t_min, c
 {
     const uint32_t cap = sc.stack_slots;
     if (W == 4u) {
-        const bool blas = (F & kHasMeshes) && !tr.in_tlas;
+        const bool blas = (F & kHasMeshes) && tr.blas_top != kInTlas;
         const float4 *nd = (blas ? sc.blas4 : sc.tlas4) + 8u * tr.addr;
         if (bvh4_node(nd, stack, stride, cap, t_min, tr)) return true;
-        return trav_pop<F>(sc, world, stack, stride, tr);
+        return trav_pop<F>(stack, stride, tr);
     }
     const float4 *node = sc.nodes2 + 4u * tr.addr;
     float4 n0 = node[0], n1 = node[1], n2 = node[2], n3 = node[3];
@@ -418,13 +418,13 @@ __device__ __forceinline__ bool trav_internal(const DevScene &sc, float t_min, c
                             tr.ox, t_min, limit, rn);
     // both hit: one child is next, the other waits on the stack (in the
     // reference's order the left one)
-    const bool left_first = !r || (ORD && sc.ordered != 0u && l && ln < rn);
+    const bool left_first = !r | (ORD & (sc.ordered != 0u) & l & (ln < rn));
     if (l && r && tr.top < cap) stack[(tr.top++) * stride] = left_first ? as_u32(n1.w) : as_u32(n0.w);
     if (l || r) {
         tr.addr = left_first ? as_u32(n0.w) : as_u32(n1.w);
         return true;
     }
-    return trav_pop<F>(sc, world, stack, stride, tr);
+    return trav_pop<F>(stack, stride, tr);
 }
 
 template <uint32_t F, uint32_t W, bool ORD>
@@ -433,7 +433,7 @@ __device__ __forceinline__ bool trav_leaf(const DevScene &sc, float t_min, const
 {
     const uint32_t cap = sc.stack_slots;
     const uint32_t idx = tr.addr & ~kLeafRef;
-    const float4 *base = W == 2u ? sc.nodes2 : ((F & kHasMeshes) && !tr.in_tlas ? sc.blas2 : sc.tlas_leaves);
+    const float4 *base = W == 2u ? sc.nodes2 : ((F & kHasMeshes) && tr.blas_top != kInTlas ? sc.blas2 : sc.tlas_leaves);
     const float4 *node = base + 4u * idx;
     float4 n0 = node[0], n1 = node[1], n2 = node[2], n3 = node[3];
     // Keep the four 16-byte loads of the node together ahead of the type
@@ -467,8 +467,7 @@ __device__ __forceinline__ bool trav_leaf(const DevScene &sc, float t_min, const
         if constexpr (ORD)
             (void)aabb_hit(make_float3(n0.x, n0.y, n0.z), make_float3(n1.x, n1.y, n1.z), tr.inv, tr.ox, t_min,
                            tr.t_max, tr.mesh_near);
-        tr.in_tlas = false;
-        if (tr.top < cap) stack[(tr.top++) * stride] = kFinishedTraverseBlas;
+        tr.blas_top = tr.top;
         tr.inv_tid = as_u32(n3.w) * 2u;
         tr.material_index = as_u32(n1.w);
         tr.ray = xform_ray(sc.transforms + 4u * tr.inv_tid, world);
@@ -504,7 +503,7 @@ __device__ __forceinline__ bool trav_leaf(const DevScene &sc, float t_min, const
             trav_behind(sc, tr, t);
         }
     }
-    return trav_pop<F>(sc, world, stack, stride, tr);
+    return trav_pop<F>(stack, stride, tr);
 }
 
 // The ray of a finished ordered search once more, in the reference's order
