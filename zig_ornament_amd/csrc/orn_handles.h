@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "../../include/ornament_hip.h"
+#include "orn_stage.h"
 #include "orn_trace.h"
 
 // Handles are reference counted: a scene holds its context and a target its
@@ -19,6 +20,7 @@ struct orn_ctx {
     char arch[64];  // gcnArchName, the autotuner's cache key
     int compute_units;
     int refs;
+    orn_rt::HostStage stage;
 };
 
 struct orn_device_scene {
@@ -65,6 +67,7 @@ inline void release_ctx(orn_ctx *c)
     if (--c->refs > 0) return;
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
+    c->stage.release();
     (void)hipStreamDestroy(c->stream);
     delete c;
 }
@@ -81,6 +84,21 @@ inline void release_scene(orn_device_scene *s)
 }
 
 inline orn_status from_hip(hipError_t e) { return e == hipSuccess ? ORN_OK : static_cast<orn_status>(e); }
+
+// Blocking copies on the context's stream (HostStage).
+inline hipError_t copy_to_host(orn_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    std::lock_guard<std::mutex> lock(c->stage.mutex);
+    return c->stage.to_host(dst, src, bytes, c->device, c->stream);
+}
+inline hipError_t copy_to_device(orn_ctx *c, void *dst, const void *src, size_t bytes)
+{
+    std::lock_guard<std::mutex> lock(c->stage.mutex);
+    const hipError_t e = c->stage.to_device(dst, src, bytes, HostStage::kPart, c->stream,
+                                            [](size_t, size_t) { return hipSuccess; });
+    const hipError_t w = hipStreamSynchronize(c->stream);
+    return e != hipSuccess ? e : w;
+}
 
 inline uint32_t blocks_for(uint32_t n, uint32_t b) { return (n + b - 1) / b; }
 

@@ -1476,17 +1476,24 @@ hipError_t train_gradients(orn_nrc *n, const NrcRecord *buf, const uint32_t *cou
 
 // The second half: MLP and grid gradients from train_gradients' output,
 // stored or applied (the only kernels of a step that write the network).
-hipError_t apply_gradients(orn_nrc *n, const uint32_t *count_ptr, uint32_t count_max, uint32_t batch, GradMode mode,
-                           hipStream_t st)
+hipError_t apply_mlp_gradients(orn_nrc *n, const uint32_t *count_ptr, uint32_t count_max, uint32_t batch,
+                               GradMode mode, hipStream_t st)
 {
     const uint32_t groups = blocks_for(batch, kTileRows);
     if (groups > n->partial_groups) return hipErrorInvalidValue;
-    const AdamStep a = adam_step(n);
     nrc_mlp_kernel<<<kMlpParams / 64u, 64u * kMlpSlices, 0, st>>>(n->partials, groups, count_ptr, count_max, batch,
-                                                                 a, n->mlp, n->mlp_grad, n->mlp_m, n->mlp_v,
-                                                                 n->mlp_wt, mode);
+                                                                 adam_step(n), n->mlp, n->mlp_grad, n->mlp_m,
+                                                                 n->mlp_v, n->mlp_wt, mode);
+    return hipGetLastError();
+}
+
+hipError_t apply_gradients(orn_nrc *n, const uint32_t *count_ptr, uint32_t count_max, uint32_t batch, GradMode mode,
+                           hipStream_t st)
+{
+    const hipError_t e = apply_mlp_gradients(n, count_ptr, count_max, batch, mode, st);
+    if (e != hipSuccess) return e;
     GridUpdate up;
-    up.a = a;
+    up.a = adam_step(n);
     up.w = n->grid_w;
     up.m = n->grid_m;
     up.v = n->grid_v;
@@ -1687,10 +1694,9 @@ orn_status orn_nrc_get_params(orn_nrc *n, float *mlp, size_t mlp_len, float *gri
     if (!n) return ORN_ERROR_INVALID_HANDLE;
     if ((mlp && mlp_len < kMlpParams) || (grid && grid_len < n->grid_params)) return ORN_ERROR_SIZE_MISMATCH;
     ORN_TRY(hipSetDevice(n->scene->ctx->device));
-    hipStream_t st = n->scene->ctx->stream;
-    if (mlp) ORN_TRY(hipMemcpyAsync(mlp, n->mlp, kMlpParams * 4, hipMemcpyDeviceToHost, st));
-    if (grid) ORN_TRY(hipMemcpyAsync(grid, n->grid_w, size_t(n->grid_params) * 4, hipMemcpyDeviceToHost, st));
-    ORN_TRY(hipStreamSynchronize(st));
+    orn_ctx *ctx = n->scene->ctx;
+    if (mlp) ORN_TRY(copy_to_host(ctx, mlp, n->mlp, kMlpParams * 4));
+    if (grid) ORN_TRY(copy_to_host(ctx, grid, n->grid_w, size_t(n->grid_params) * 4));
     return ORN_OK;
 }
 
@@ -1700,8 +1706,9 @@ orn_status orn_nrc_set_params(orn_nrc *n, const float *mlp, size_t mlp_len, cons
     if ((mlp && mlp_len != kMlpParams) || (grid && grid_len != n->grid_params)) return ORN_ERROR_SIZE_MISMATCH;
     ORN_TRY(hipSetDevice(n->scene->ctx->device));
     hipStream_t st = n->scene->ctx->stream;
-    if (mlp) ORN_TRY(hipMemcpyAsync(n->mlp, mlp, kMlpParams * 4, hipMemcpyHostToDevice, st));
-    if (grid) ORN_TRY(hipMemcpyAsync(n->grid_w, grid, size_t(n->grid_params) * 4, hipMemcpyHostToDevice, st));
+    orn_ctx *ctx = n->scene->ctx;
+    if (mlp) ORN_TRY(copy_to_device(ctx, n->mlp, mlp, kMlpParams * 4));
+    if (grid) ORN_TRY(copy_to_device(ctx, n->grid_w, grid, size_t(n->grid_params) * 4));
     ORN_TRY(refresh_params(n, st));
     ORN_TRY(hipStreamSynchronize(st));
     return ORN_OK;
@@ -1713,26 +1720,30 @@ orn_status orn_nrc_query(orn_nrc *n, const orn_nrc_record *records, size_t count
     if (!records || !rgb || count == 0 || count > (1u << 24)) return ORN_ERROR_INVALID_VALUE;
     ORN_TRY(hipSetDevice(n->scene->ctx->device));
     hipStream_t st = n->scene->ctx->stream;
-    NrcRecord *d_rec = nullptr;
-    float *d_out = nullptr, *d_in = nullptr;
-    hipError_t e = hipMalloc(&d_rec, count * sizeof(NrcRecord));
-    if (!e) e = hipMalloc(&d_out, count * 12);
-    if (!e && inputs) e = hipMalloc(&d_in, count * kIn * 4);
-    if (!e) e = hipMemcpyAsync(d_rec, records, count * sizeof(NrcRecord), hipMemcpyHostToDevice, st);
+    orn_ctx *ctx = n->scene->ctx;
+    HostStage &stage = ctx->stage;
+    std::lock_guard<std::mutex> lock(stage.mutex);
+    void *ws = nullptr;
+    bool own = false;
+    hipError_t e = stage.workspace(count * (sizeof(NrcRecord) + 12 + (inputs ? kIn * 4 : 0)), &ws, &own);
     if (!e) {
-        const uint32_t tiles = blocks_for(static_cast<uint32_t>(count), kTileRows);
-        nrc_infer_kernel<<<std::min<uint32_t>(blocks_for(tiles * 4u, kInferWaves), 1024u), 64u * kInferWaves, 0, st>>>(
-            n->grid, reinterpret_cast<const __half2 *>(n->grid_half), n->mlp_wt, d_rec, nullptr,
-            static_cast<uint32_t>(count), 0, d_out, PixelSink{}, d_in);
-        e = hipGetLastError();
+        NrcRecord *d_rec = static_cast<NrcRecord *>(ws);
+        float *d_in = inputs ? reinterpret_cast<float *>(d_rec + count) : nullptr;
+        float *d_out = reinterpret_cast<float *>(d_rec + count) + (inputs ? count * kIn : 0);
+        e = stage.to_device(d_rec, records, count * sizeof(NrcRecord), HostStage::kPart, st,
+                            [](size_t, size_t) { return hipSuccess; });
+        if (!e) {
+            const uint32_t tiles = blocks_for(static_cast<uint32_t>(count), kTileRows);
+            nrc_infer_kernel<<<std::min<uint32_t>(blocks_for(tiles * 4u, kInferWaves), 1024u), 64u * kInferWaves, 0,
+                               st>>>(n->grid, reinterpret_cast<const __half2 *>(n->grid_half), n->mlp_wt, d_rec,
+                                     nullptr, static_cast<uint32_t>(count), 0, d_out, PixelSink{}, d_in);
+            e = hipGetLastError();
+        }
+        if (!e) e = stage.to_host(rgb, d_out, count * 12, ctx->device, st);
+        if (!e && inputs) e = stage.to_host(inputs, d_in, count * kIn * 4, ctx->device, st);
     }
-    if (!e) e = hipMemcpyAsync(rgb, d_out, count * 12, hipMemcpyDeviceToHost, st);
-    if (!e && inputs) e = hipMemcpyAsync(inputs, d_in, count * kIn * 4, hipMemcpyDeviceToHost, st);
-    if (!e) e = hipStreamSynchronize(st);
     (void)hipStreamSynchronize(st);
-    if (d_rec) (void)hipFree(d_rec);
-    if (d_out) (void)hipFree(d_out);
-    if (d_in) (void)hipFree(d_in);
+    if (own && ws) (void)hipFree(ws);
     return from_hip(e);
 }
 
@@ -1745,25 +1756,45 @@ static orn_status host_batch(orn_nrc *n, const orn_nrc_record *records, size_t c
     if (grid_grad && grid_len < n->grid_params) return ORN_ERROR_SIZE_MISMATCH;
     ORN_TRY(hipSetDevice(n->scene->ctx->device));
     hipStream_t st = n->scene->ctx->stream;
+    orn_ctx *ctx = n->scene->ctx;
     const uint32_t c = static_cast<uint32_t>(count);
-    ORN_TRY(hipMemcpyAsync(n->train_recs, records, count * sizeof(NrcRecord), hipMemcpyHostToDevice, st));
-    nrc_zero_kernel<<<1, 32, 0, st>>>(n->loss, 4);
-    if (update) {
-        n->step++;
-        ORN_TRY(gradients(n, n->train_recs, nullptr, c, 0u, c, kUpdate, st));
-    } else {
+    HostStage &stage = ctx->stage;
+    std::lock_guard<std::mutex> lock(stage.mutex);
+    auto run = [&]() -> hipError_t {
+        hipError_t e = stage.to_device(n->train_recs, records, count * sizeof(NrcRecord),
+                                       HostStage::kPart, st,
+                                       [](size_t, size_t) { return hipSuccess; });
+        if (e) return e;
+        nrc_zero_kernel<<<1, 32, 0, st>>>(n->loss, 4);
+        if (update) {
+            n->step++;
+            return gradients(n, n->train_recs, nullptr, c, 0u, c, kUpdate, st);
+        }
+        if (!grid_grad) {  // the grid's gradient was not asked for: the weights' alone
+            e = train_gradients(n, n->train_recs, nullptr, c, 0u, c, st);
+            return e ? e : apply_mlp_gradients(n, nullptr, c, c, kGradient, st);
+        }
         // entries of dense levels past their lattice are never written by the gradient kernel
         const uint64_t gp = n->grid_params;
         nrc_zero_kernel<<<static_cast<uint32_t>((gp + 255) / 256), 256, 0, st>>>(n->grid_grad, gp);
-        ORN_TRY(gradients(n, n->train_recs, nullptr, c, 0u, c, kGradient, st));
-        if (mlp_grad) ORN_TRY(hipMemcpyAsync(mlp_grad, n->mlp_grad, kMlpParams * 4, hipMemcpyDeviceToHost, st));
-        if (grid_grad)
-            ORN_TRY(hipMemcpyAsync(grid_grad, n->grid_grad, size_t(n->grid_params) * 4, hipMemcpyDeviceToHost, st));
-    }
+        return gradients(n, n->train_recs, nullptr, c, 0u, c, kGradient, st);
+    };
+    hipError_t e = run();
+    if (!e && !update && grid_grad) e = stage.to_host(grid_grad, n->grid_grad, size_t(n->grid_params) * 4, ctx->device, st);
+    // the loss and the weights' gradient behind one wait
     float l = 0.0f;
-    ORN_TRY(hipMemcpyAsync(&l, n->loss, 4, hipMemcpyDeviceToHost, st));
-    ORN_TRY(hipStreamSynchronize(st));
-    if (loss) *loss = l;
+    static_assert(kMlpParams * 4 + 4 <= HostStage::kBytes, "gradient and loss fit the pinned buffer");
+    char *pin = stage.pinned();
+    float *h_loss = pin ? reinterpret_cast<float *>(pin) : &l;
+    float *h_grad = pin ? h_loss + 1 : mlp_grad;
+    const bool want = !update && mlp_grad;
+    if (!e) e = hipMemcpyAsync(h_loss, n->loss, 4, hipMemcpyDeviceToHost, st);
+    if (!e && want) e = hipMemcpyAsync(h_grad, n->mlp_grad, kMlpParams * 4, hipMemcpyDeviceToHost, st);
+    const hipError_t w = hipStreamSynchronize(st);
+    if (!e) e = w;
+    if (e) return from_hip(e);
+    if (want && pin) std::memcpy(mlp_grad, h_grad, kMlpParams * 4);
+    if (loss) *loss = *h_loss;
     return ORN_OK;
 }
 

@@ -2150,9 +2150,7 @@ static orn_status readback(orn_target *t, void *dst, const void *src, size_t ele
     const size_t n = size_t(t->width) * t->height;
     if (pixels < n) return ORN_ERROR_SIZE_MISMATCH;
     ORN_TRY(hipSetDevice(t->scene->ctx->device));
-    hipStream_t st = t->scene->ctx->stream;
-    ORN_TRY(hipMemcpyAsync(dst, src, n * elem, hipMemcpyDeviceToHost, st));
-    ORN_TRY(hipStreamSynchronize(st));
+    ORN_TRY(copy_to_host(t->scene->ctx, dst, src, n * elem));
     return ORN_OK;
 }
 
@@ -2183,12 +2181,19 @@ orn_status orn_set_state(orn_target *t, const float *accumulation, const uint32_
     const size_t n = size_t(t->width) * t->height;
     if (pixels != n) return ORN_ERROR_SIZE_MISMATCH;
     ORN_TRY(hipSetDevice(t->scene->ctx->device));
-    hipStream_t st = t->scene->ctx->stream;
-    if (accumulation) ORN_TRY(hipMemcpyAsync(t->acc, accumulation, n * sizeof(float4), hipMemcpyHostToDevice, st));
-    if (rng) ORN_TRY(hipMemcpyAsync(t->rng, rng, n * sizeof(uint32_t), hipMemcpyHostToDevice, st));
-    ORN_TRY(hipStreamSynchronize(st));
+    orn_ctx *ctx = t->scene->ctx;
+    if (accumulation) ORN_TRY(copy_to_device(ctx, t->acc, accumulation, n * sizeof(float4)));
+    if (rng) ORN_TRY(copy_to_device(ctx, t->rng, rng, n * sizeof(uint32_t)));
     return ORN_OK;
 }
+
+// Rays up to here are read from, and their hits written to, pinned host
+// memory by the kernel itself: two small copies and their waits cost more
+// than the lanes' own accesses over the link (256 rays: 53 -> 34 us).
+static constexpr size_t kDirectRays = 4096;
+// Rays per launch of a longer query, so that the next ones are copied while
+// these are traced.
+static constexpr size_t kRaysPerPiece = 131072;
 
 static orn_status trace_rays(orn_device_scene *s, float t_min, const float *rays, size_t n, orn_hit *out,
                              bool packet)
@@ -2197,33 +2202,47 @@ static orn_status trace_rays(orn_device_scene *s, float t_min, const float *rays
     if ((!rays || !out) && n) return ORN_ERROR_INVALID_VALUE;
     if (n == 0) return ORN_OK;
     if (n > 0xffffffffull) return ORN_ERROR_INVALID_VALUE;
-    ORN_TRY(hipSetDevice(s->ctx->device));
-    hipStream_t st = s->ctx->stream;
-    float *d_rays = nullptr;
-    orn_hit *d_out = nullptr;
-    hipError_t e = hipMalloc(&d_rays, n * 6 * sizeof(float));
-    if (e == hipSuccess) e = hipMalloc(&d_out, n * sizeof(orn_hit));
-    if (e == hipSuccess) e = hipMemcpyAsync(d_rays, rays, n * 6 * sizeof(float), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) {
-        DevScene ds = s->ds;
-        ds.stack_slots = s->trace_width == 4u ? s->stack_slots4 : s->traversal_slots;
-        const size_t lds = size_t(ds.stack_slots) * kBlock * sizeof(uint32_t);
-        const uint32_t blocks = blocks_for(static_cast<uint32_t>(n), kBlock);
-        if (packet) {
-            ds.stack_slots = s->stack_slots;
-            trace_packet_kernel<<<blocks, kBlock, 0, st>>>(ds, t_min, d_rays, static_cast<uint32_t>(n), d_out);
-        } else if (s->trace_width == 4u) {
-            trace_kernel<4><<<blocks, kBlock, lds, st>>>(ds, t_min, d_rays, static_cast<uint32_t>(n), d_out);
-        } else {
-            trace_kernel<2><<<blocks, kBlock, lds, st>>>(ds, t_min, d_rays, static_cast<uint32_t>(n), d_out);
-        }
-        e = hipGetLastError();
+    orn_ctx *ctx = s->ctx;
+    ORN_TRY(hipSetDevice(ctx->device));
+    hipStream_t st = ctx->stream;
+    DevScene ds = s->ds;
+    ds.stack_slots = packet ? s->stack_slots : s->trace_width == 4u ? s->stack_slots4 : s->traversal_slots;
+    const size_t lds = size_t(ds.stack_slots) * kBlock * sizeof(uint32_t);
+    auto launch = [&](const float *d_rays, size_t count, orn_hit *d_out) {
+        const uint32_t c = static_cast<uint32_t>(count), blocks = blocks_for(c, kBlock);
+        if (packet) trace_packet_kernel<<<blocks, kBlock, 0, st>>>(ds, t_min, d_rays, c, d_out);
+        else if (s->trace_width == 4u) trace_kernel<4><<<blocks, kBlock, lds, st>>>(ds, t_min, d_rays, c, d_out);
+        else trace_kernel<2><<<blocks, kBlock, lds, st>>>(ds, t_min, d_rays, c, d_out);
+        return hipGetLastError();
+    };
+    constexpr size_t kRay = 6 * sizeof(float);
+    static_assert(kDirectRays * (kRay + sizeof(orn_hit)) <= HostStage::kBytes, "direct rays and hits fit the buffer");
+    static_assert(kRaysPerPiece * kRay <= HostStage::kPart && kRaysPerPiece % kBlock == 0,
+                  "a piece of rays fits its part of the buffer");
+    std::lock_guard<std::mutex> lock(ctx->stage.mutex);
+    if (n <= kDirectRays && ctx->stage.pinned()) {
+        float *h_rays = reinterpret_cast<float *>(ctx->stage.pinned());
+        orn_hit *h_out = reinterpret_cast<orn_hit *>(ctx->stage.pinned() + kDirectRays * kRay);
+        std::memcpy(h_rays, rays, n * kRay);
+        hipError_t e = launch(h_rays, n, h_out);
+        const hipError_t w = hipStreamSynchronize(st);
+        if (e == hipSuccess) e = w;
+        if (e == hipSuccess) std::memcpy(out, h_out, n * sizeof(orn_hit));
+        return from_hip(e);
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(out, d_out, n * sizeof(orn_hit), hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    void *ws = nullptr;
+    bool own = false;
+    hipError_t e = ctx->stage.workspace(n * (kRay + sizeof(orn_hit)), &ws, &own);
+    if (e == hipSuccess) {
+        orn_hit *d_out = static_cast<orn_hit *>(ws);  // 32-byte hits first: rays after them stay aligned
+        float *d_rays = reinterpret_cast<float *>(d_out + n);
+        e = ctx->stage.to_device(d_rays, rays, n * kRay, kRaysPerPiece * kRay, st, [&](size_t at, size_t bytes) {
+            return launch(d_rays + at / sizeof(float), bytes / kRay, d_out + at / kRay);
+        });
+        if (e == hipSuccess) e = ctx->stage.to_host(out, d_out, n * sizeof(orn_hit), ctx->device, st);
+    }
     (void)hipStreamSynchronize(st);
-    if (d_rays) (void)hipFree(d_rays);
-    if (d_out) (void)hipFree(d_out);
+    if (own && ws) (void)hipFree(ws);
     return from_hip(e);
 }
 
@@ -2578,10 +2597,8 @@ orn_status batch_readback(orn_batch *b, size_t item, void *dst, const void *pool
     const size_t n = size_t(b->width[item]) * b->height[item];
     if (pixels < n) return ORN_ERROR_SIZE_MISMATCH;
     ORN_TRY(hipSetDevice(b->scene->ctx->device));
-    hipStream_t st = b->scene->ctx->stream;
     const char *src = static_cast<const char *>(pool) + size_t(b->px_base[item]) * elem;
-    ORN_TRY(hipMemcpyAsync(dst, src, n * elem, hipMemcpyDeviceToHost, st));
-    ORN_TRY(hipStreamSynchronize(st));
+    ORN_TRY(copy_to_host(b->scene->ctx, dst, src, n * elem));
     return ORN_OK;
 }
 
@@ -2794,12 +2811,10 @@ orn_status orn_batch_set_state(orn_batch *b, size_t item, const float *accumulat
     const size_t n = size_t(b->width[item]) * b->height[item];
     if (pixels != n) return ORN_ERROR_SIZE_MISMATCH;
     ORN_TRY(hipSetDevice(b->scene->ctx->device));
-    hipStream_t st = b->scene->ctx->stream;
+    orn_ctx *ctx = b->scene->ctx;
     const size_t at = b->px_base[item];
-    if (accumulation)
-        ORN_TRY(hipMemcpyAsync(b->acc + at, accumulation, n * sizeof(float4), hipMemcpyHostToDevice, st));
-    if (rng) ORN_TRY(hipMemcpyAsync(b->rng + at, rng, n * sizeof(uint32_t), hipMemcpyHostToDevice, st));
-    ORN_TRY(hipStreamSynchronize(st));
+    if (accumulation) ORN_TRY(copy_to_device(ctx, b->acc + at, accumulation, n * sizeof(float4)));
+    if (rng) ORN_TRY(copy_to_device(ctx, b->rng + at, rng, n * sizeof(uint32_t)));
     return ORN_OK;
 }
 

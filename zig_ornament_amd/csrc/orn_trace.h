@@ -431,7 +431,6 @@ template <uint32_t F, uint32_t W, bool ORD>
 __device__ __forceinline__ bool trav_leaf(const DevScene &sc, float t_min, const Ray &world,
                                           uint32_t *stack, uint32_t stride, Traversal &tr)
 {
-    const uint32_t cap = sc.stack_slots;
     const uint32_t idx = tr.addr & ~kLeafRef;
     const float4 *base = W == 2u ? sc.nodes2 : ((F & kHasMeshes) && tr.blas_top != kInTlas ? sc.blas2 : sc.tlas_leaves);
     const float4 *node = base + 4u * idx;
