@@ -55,6 +55,8 @@ constexpr uint32_t kQueueStride = 32;
 // end (a quarter instead of a 64th: a 16-image batch 12.4 -> 15 ms). Only for
 // whole pixels: a wave must not hold a split pixel's job back while all its
 // lanes wait for jobs that other waves hold back.
+// Most lanes of a sparse wave, and the step they come in (launch_render_k).
+constexpr uint32_t kSparseLanes = 8, kLaneStep = 4;
 constexpr uint32_t kAheadShare = 64, kAheadMost = 64;
 constexpr uint32_t kQueueWords = kXcds * kQueueStride;
 constexpr uint32_t kMaxStack = 63;  // the reference's private stack has 64 slots
@@ -75,6 +77,7 @@ struct KernelParams {
     uint32_t epoch;         // tag of this launch in the stage words (single image)
     uint32_t split_pct;     // percentage of each band's pixels that are split
     uint32_t pixels;        // pixels in the pixel buffers (at most 2^28)
+    uint32_t lanes;         // lanes of each wave that take pixels (the rest stay idle)
     const uint32_t *order;  // queue position -> tile-pixel of the band, or null: tile order
     uint32_t *cost;         // per-pixel job time to record, or null
 };
@@ -278,7 +281,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
     Traversal tr;
     tr.addr = kLeafRef;  // a lane that is not traversing holds a leaf-flagged reference
     tr.redo = false;
-    uint32_t mode = kWaiting;
+    uint32_t mode = lane < kp.lanes ? kWaiting : kDone;
     bool need_pixel = true;
     bool blocked = false;  // holds a job whose predecessor has not finished
     // per-image values a lane keeps while it works on a pixel (BATCH); a
@@ -1301,7 +1304,8 @@ struct LaunchArgs {
 
 // One instantiation per combination of scene features.
 // Persistent grid: workgroups_per_cu per compute unit (0: as many as can be
-// resident at once), a multiple of the XCD count, at most one per tile.
+// resident at once), a multiple of the XCD count; at most one per tile when
+// the waves are full.
 template <uint32_t F, uint32_t W, bool BATCH, bool POOL>
 hipError_t launch_render_k(uint32_t per_cu, uint32_t cus, size_t lds, hipStream_t st, const DevScene &ds,
                            const LaunchArgs &a)
@@ -1316,11 +1320,28 @@ hipError_t launch_render_k(uint32_t per_cu, uint32_t cus, size_t lds, hipStream_
         }
         per_cu = static_cast<uint32_t>(blocks);
     }
-    uint32_t grid = cus * per_cu;
-    grid = std::min(grid, blocks_for(a.total_tiles, kXcds) * kXcds);
-    grid = std::max(kXcds, grid / kXcds * kXcds);
+    uint32_t grid = std::max(kXcds, cus * per_cu / kXcds * kXcds);
+    // A pixel is one lane's work from its first sample to its last, so an image
+    // of fewer pixels than lanes leaves the choice between few full waves and
+    // many sparse ones. In sparse waves a lane waits for fewer others at leaf
+    // and shading rounds, but those rounds are issued once per wave, so the
+    // SIMDs must have the issue slots: up to 8 lanes of every resident wave.
+    // 8 spp, full -> sparse: instanced icospheres 64x64 1.64 -> 0.92 ms,
+    // 160x160 1.91 -> 1.36; random spheres 128x128 0.97 -> 0.75, 160x160 0.94 ->
+    // 0.85; Cornell box (every path bounces to its full depth) 96x96 0.86 ->
+    // 0.65, 181x181 0.85 -> 0.87. Above that the box loses more than the others
+    // gain (200x200 at 12 lanes: 0.83 -> 0.96, icospheres 1.83 -> 1.50).
+    KernelParams kp = a.kp;
+    const uint32_t per_wave = blocks_for(kp.pixels, grid * (kBlock / 64u));
+    kp.lanes = POOL || per_wave > kSparseLanes ? 64u : blocks_for(per_wave, kLaneStep) * kLaneStep;
+    if (kp.lanes == 64u) {
+        grid = std::min(grid, blocks_for(a.total_tiles, kXcds) * kXcds);
+    } else {
+        kp.regroup = std::max(1u, kp.regroup * kp.lanes / 64u);
+        kp.leaf_regroup = std::max(1u, kp.leaf_regroup * kp.lanes / 64u);
+    }
     render_kernel<F, W, BATCH, POOL>
-        <<<grid, kBlock, lds, st>>>(ds, a.kp, a.items, a.work, a.acc, a.rng, a.stage, a.queues);
+        <<<grid, kBlock, lds, st>>>(ds, kp, a.items, a.work, a.acc, a.rng, a.stage, a.queues);
     return hipGetLastError();
 }
 
