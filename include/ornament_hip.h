@@ -227,6 +227,8 @@ orn_status orn_render_async(orn_target *target, const orn_constant_params *param
                             uint32_t iterations);
 orn_status orn_target_wait(orn_target *target);
 /* Launch tuning of a target's render kernel; any value gives the same image.
+ * Until one is set (or found by the autotuner) the library picks the shape of
+ * every launch itself; orn_target_get_tuning then returns the defaults below.
  * regroup_lanes (1..64): a wave interrupts BVH traversal for a shading round
  *   once this many of its 64 lanes have finished their ray (default 48).
  * workgroups_per_cu (0..64): persistent 256-lane workgroups launched per
@@ -293,7 +295,7 @@ orn_status orn_target_get_tuning(orn_target *target, orn_tuning *tuning);
  * for split pixels) is a library-owned device array, one per device, sized
  * for ORN_RENDER_SCRATCH_PIXELS pixels (8 MiB) and held until the process
  * ends; larger images return ORN_ERROR_SCRATCH_TOO_SMALL before anything is
- * enqueued. `tuning` may be NULL (the default tuning). `stream` is a
+ * enqueued. `tuning` may be NULL (the library picks). `stream` is a
  * hipStream_t of the scene's device, or NULL for the device context's own
  * stream. The call returns once the work is enqueued. Every call on a device
  * uses the same scratch: calls whose work overlaps in time on one device (on

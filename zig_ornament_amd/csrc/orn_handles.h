@@ -41,6 +41,7 @@ struct orn_device_scene {
 struct orn_target {
     orn_device_scene *scene;
     orn_tuning tuning;
+    bool tuned = false;  // `tuning` was set; until then the library picks
     uint32_t width, height;
     float4 *fb;
     float4 *acc;
