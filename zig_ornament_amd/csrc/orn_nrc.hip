@@ -960,7 +960,7 @@ __device__ __forceinline__ f3 continue_path(const DevScene &sc, const orn_consta
 {
     for (uint32_t b = b0; b < p.depth; b++) {
         Hit h{};
-        if (!bvh_hit<F, 2, kNodeSteps>(sc, p.ray_cast_epsilon, ray, stack, kBlock, h)) return thr * sky(ray.d);
+        if (!bvh_hit<F, bvh2_format(F), kNodeSteps>(sc, p.ray_cast_epsilon, ray, stack, kBlock, h)) return thr * sky(ray.d);
         Ray next;
         f3 w;
         if (shade<F>(sc, p.textures_count, 0u, ray, normalize(ray.d), h, rng, next, w)) {
@@ -1016,7 +1016,7 @@ __global__ __launch_bounds__(kBlock) void nrc_paths_kernel(DevScene sc, orn_cons
         bool done = false;
         for (uint32_t b = 0; b < p.depth && !done; b++) {
             Hit h{};
-            if (!bvh_hit<F, 2, kNodeSteps>(sc, p.ray_cast_epsilon, ray, stack, kBlock, h)) {
+            if (!bvh_hit<F, bvh2_format(F), kNodeSteps>(sc, p.ray_cast_epsilon, ray, stack, kBlock, h)) {
                 color = thr * sky(ray.d);
                 done = true;
                 break;
@@ -1096,7 +1096,7 @@ __global__ __launch_bounds__(kBlock) void nrc_primary_kernel(DevScene sc, orn_co
     if constexpr (kPacket) {
         hit = bvh_hit_packet<F>(sc, p.ray_cast_epsilon, ray, active && p.depth > 0u, sc.stack_slots, h);
     } else if (active && p.depth > 0u) {
-        hit = bvh_hit<F, 2, kNodeSteps>(sc, p.ray_cast_epsilon, ray, lds_stack + threadIdx.x, kBlock, h);
+        hit = bvh_hit<F, bvh2_format(F), kNodeSteps>(sc, p.ray_cast_epsilon, ray, lds_stack + threadIdx.x, kBlock, h);
     }
     bool query = false;
     NrcRecord rc;
@@ -1226,7 +1226,7 @@ __global__ __launch_bounds__(kBlock) void nrc_train_paths_kernel(DevScene sc, or
         Ray ray = camera_ray(p, pix % p.width, pix / p.width, rng);
         for (uint32_t b = 0; b <= k && b < p.depth; b++) {
             Hit h{};
-            if (!bvh_hit<F, 2, kNodeSteps>(sc, p.ray_cast_epsilon, ray, stack, kBlock, h)) break;
+            if (!bvh_hit<F, bvh2_format(F), kNodeSteps>(sc, p.ray_cast_epsilon, ray, stack, kBlock, h)) break;
             const Surface s = surface<F>(sc, p.textures_count, 0u, ray, h);
             Ray next;
             f3 w;
@@ -1396,7 +1396,7 @@ void launch_train_paths(orn_nrc *n, const DevScene &ds, const orn_constant_param
 }
 
 #define ORN_NRC_DISPATCH(fn, features, ...)        \
-    switch ((features) & 7u) {                     \
+    switch ((features) & 15u) {                    \
     case 0: fn<0>(__VA_ARGS__); break;             \
     case 1: fn<1>(__VA_ARGS__); break;             \
     case 2: fn<2>(__VA_ARGS__); break;             \
@@ -1404,7 +1404,15 @@ void launch_train_paths(orn_nrc *n, const DevScene &ds, const orn_constant_param
     case 4: fn<4>(__VA_ARGS__); break;             \
     case 5: fn<5>(__VA_ARGS__); break;             \
     case 6: fn<6>(__VA_ARGS__); break;             \
-    default: fn<7>(__VA_ARGS__); break;            \
+    case 7: fn<7>(__VA_ARGS__); break;             \
+    case 8: fn<8>(__VA_ARGS__); break;             \
+    case 9: fn<9>(__VA_ARGS__); break;             \
+    case 10: fn<10>(__VA_ARGS__); break;           \
+    case 11: fn<11>(__VA_ARGS__); break;           \
+    case 12: fn<12>(__VA_ARGS__); break;           \
+    case 13: fn<13>(__VA_ARGS__); break;           \
+    case 14: fn<14>(__VA_ARGS__); break;           \
+    default: fn<15>(__VA_ARGS__); break;           \
     }
 
 void free_nrc(orn_nrc *n)

@@ -257,7 +257,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                                                         uint32_t *__restrict__ stage,
                                                         uint32_t *__restrict__ queues)
 {
-    constexpr bool kOrdered = W == 2u;
+    constexpr uint32_t kFormat = W == 4u ? 4u : bvh2_format(F);  // of the nodes
     extern __shared__ uint32_t lds_stack[];
     uint32_t *stack = lds_stack + threadIdx.x;
     const uint32_t lane = threadIdx.x % 64u;
@@ -440,7 +440,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
     bool shade_all = false;  // POOL: this iteration's workgroup-wide shading decision
     for (;;) {
         if constexpr (POOL) {
-            static_assert(!(F & kHasMeshes) && W == 2u && !BATCH, "pooled traversal: spheres, BVH2, one image");
+            static_assert(!(F & kHasMeshes) && kFormat == 2u && !BATCH, "pooled traversal: spheres, BVH2, one image");
             __shared__ float p_f[7][kBlock];  // inv xyz, ox xyz, t_cull of each slot
             __shared__ uint32_t p_addr[kBlock], p_top[kBlock];
             __shared__ uint64_t p_mask[kBlock / 64u];
@@ -496,11 +496,12 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                     wt.inv = mk(p_f[0][slot], p_f[1][slot], p_f[2][slot]);
                     wt.ox = mk(p_f[3][slot], p_f[4][slot], p_f[5][slot]);
                     wt.t_cull = p_f[6][slot];
+                    trav_signs(wt);
                     wt.addr = p_addr[slot];
                     wt.top = p_top[slot];
                 }
                 for (uint32_t k = 0; k < node_steps; k++) {
-                    if (!(wt.addr & kLeafRef) && !trav_internal<F, W, kOrdered>(sc, t_min(), ray, lds_stack + slot, kBlock, wt))
+                    if (!(wt.addr & kLeafRef) && !trav_internal<F, kFormat>(sc, t_min(), ray, lds_stack + slot, kBlock, wt))
                         wt.addr = kDoneRef;
                 }
                 if (mine) {
@@ -523,7 +524,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
             // of at least `leaf_regroup` lanes. An unflagged tr.addr implies
             // mode == kTraverse: lanes that stop traversing take kLeafRef.
             for (uint32_t k = 0; k < node_steps; k++) {
-                if (!(tr.addr & kLeafRef) && !trav_internal<F, W, kOrdered>(sc, t_min(), ray, stack, kBlock, tr)) {
+                if (!(tr.addr & kLeafRef) && !trav_internal<F, kFormat>(sc, t_min(), ray, stack, kBlock, tr)) {
                     mode = kWaiting;
                     tr.addr = kLeafRef;
                 }
@@ -535,7 +536,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
         const uint64_t at_leaf = tracing & ~at_inner;
         if (at_leaf != 0u && (static_cast<uint32_t>(__popcll(at_leaf)) >= leaf_regroup || at_inner == 0u)) {
             if (mode == kTraverse && (tr.addr & kLeafRef) &&
-                !trav_leaf<F, W, kOrdered>(sc, t_min(), ray, stack, kBlock, tr)) {
+                !trav_leaf<F, kFormat>(sc, t_min(), ray, stack, kBlock, tr)) {
                 mode = kWaiting;
                 tr.addr = kLeafRef;
             }
@@ -573,7 +574,7 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
                     begin_job();
                 }
             } else {
-                if (kOrdered && tr.redo)
+                if (is_search_format(kFormat) && tr.redo)
                     trav_redo<F>(sc, BATCH ? items[item].root2 : sc.tlas2_root, t_min(), ray, stack, kBlock, tr);
                 bounce++;
                 // each lane's outcome first, then one next_traversal for all
@@ -911,7 +912,7 @@ __global__ __launch_bounds__(kBlock) void trace_kernel(DevScene sc, float t_min,
     r.o = mk(rays[6u * i], rays[6u * i + 1u], rays[6u * i + 2u]);
     r.d = mk(rays[6u * i + 3u], rays[6u * i + 4u], rays[6u * i + 5u]);
     Hit h{};
-    const bool hit = bvh_hit<kHasSpheres | kHasMeshes, W>(sc, t_min, r, lds_stack + threadIdx.x, kBlock, h);
+    const bool hit = bvh_hit<W == 2u ? kHasSpheres : kHasSpheres | kHasMeshes, W>(sc, t_min, r, lds_stack + threadIdx.x, kBlock, h);
     orn_hit o{};
     o.hit = hit ? 1u : 0u;
     if (hit) {
@@ -1368,7 +1369,7 @@ template <uint32_t F, uint32_t W, bool BATCH>
 hipError_t launch_render_f(uint32_t per_cu, uint32_t cus, size_t lds, hipStream_t st, const DevScene &ds,
                            const LaunchArgs &a)
 {
-    if constexpr (!(F & kHasMeshes) && W == 2u && !BATCH)
+    if constexpr (!(F & (kHasMeshes | kNoSearchTree)) && W == 2u && !BATCH)
         if (a.pool) return launch_render_k<F, W, BATCH, true>(per_cu, cus, lds, st, ds, a);
     return launch_render_k<F, W, BATCH, false>(per_cu, cus, lds, st, ds, a);
 }
@@ -1377,11 +1378,14 @@ template <bool BATCH>
 hipError_t launch_render(uint32_t features, uint32_t width, uint32_t per_cu, uint32_t cus, size_t lds,
                          hipStream_t st, const DevScene &ds, const LaunchArgs &a)
 {
-#define ORN_CASE(F)                                                                      \
-    case F:                                                                              \
+#define ORN_CASE(F)                                                              \
+    case F:                                                                      \
         return width == 4u ? launch_render_f<F, 4, BATCH>(per_cu, cus, lds, st, ds, a)  \
-                           : launch_render_f<F, 2, BATCH>(per_cu, cus, lds, st, ds, a);
-    switch (features & 7u) {
+                           : launch_render_f<F, 2, BATCH>(per_cu, cus, lds, st, ds, a); \
+    case F | kNoSearchTree:                                                      \
+        return width == 4u ? launch_render_f<F, 4, BATCH>(per_cu, cus, lds, st, ds, a)  \
+                           : launch_render_f<F | kNoSearchTree, 2, BATCH>(per_cu, cus, lds, st, ds, a);
+    switch (features & 15u) {
         ORN_CASE(0u)
         ORN_CASE(1u)
         ORN_CASE(2u)
@@ -1550,22 +1554,26 @@ void fill_sphere_leaves(const orn_scene_desc *d, std::vector<orn_bvh_node> &node
 }
 
 // The search tree of the ordered traversal (orn_sah.h, orn_trace.h) over the
-// leaves of flagged BVH2 copies: its internal nodes (and a copy of every mesh
-// leaf that enters its BLAS's search tree) are appended to `tlas` and `blas`.
+// leaves of flagged BVH2 copies. A copy of every mesh leaf that enters its
+// BLAS's search tree is appended to `tlas`.
 // Rays get the reference's hits only if its boxes are what its build makes
 // them: finite, each containing the boxes below it, a triangle's own spanning
 // its vertices, every node under one parent. Arrays that are not so keep the
 // reference's order throughout (build returns false and leaves them alone).
 class SearchTree {
 public:
+    std::vector<uint32_t> nodes;  // TLAS trees, then BLAS trees, in the given format
     std::vector<uint32_t> roots;  // search root reference of each TLAS root
     uint32_t slots = 1;           // traversal stack entries it needs, in any order of the children
 
-    bool build(const orn_scene_desc *d, const uint32_t *tlas_roots, size_t n_roots, std::vector<orn_bvh_node> &tlas,
-               std::vector<orn_bvh_node> &blas)
+    // `format`: bvh2_format() of the scene's launches, 2 or 3.
+    explicit SearchTree(uint32_t format) : format_(format) {}
+
+    bool build(const orn_scene_desc *d, const uint32_t *tlas_roots, size_t n_roots, std::vector<orn_bvh_node> &tlas)
     {
         if (!nested(d->tlas_nodes, d->tlas_nodes_len) || !nested(d->blas_nodes, d->blas_nodes_len)) return false;
-        std::vector<orn_bvh_node> t = tlas, b = blas;
+        std::vector<orn_bvh_node> t = tlas;
+        std::vector<uint32_t> b;  // the BLAS trees, from place 0 until they join the TLAS's
         std::vector<uint32_t> blas_root(d->blas_nodes_len, kEmptyRef), blas_slots(d->blas_nodes_len, 0u);
         std::vector<orn_sah::Leaf> leaves, blas_leaves;
         std::vector<uint32_t> below(t.size(), 0u);  // stack entries a TLAS leaf's BLAS needs
@@ -1594,17 +1602,26 @@ public:
                 nd.left_or_custom_id = blas_root[r];
                 l.ref = kLeafRef | static_cast<uint32_t>(t.size());
                 t.push_back(nd);
-                below.push_back(1u + blas_slots[r]);  // the marker, then the BLAS
+                below.push_back(1u + blas_slots[r]);
             }
             uint32_t root = kEmptyRef;
-            if (!grow(leaves, t, &root)) return false;
-            below.resize(t.size(), 0u);
+            if (!grow(leaves, nodes, &root)) return false;
             roots.push_back(root);
-            slots = std::max(slots, pending(t, root, &below));
+            slots = std::max(slots, pending(nodes, root, &below));
         }
-        if (slots > kMaxStack || t.size() >= kLeafRef || b.size() >= kLeafRef) return false;
+        if (slots > kMaxStack || t.size() >= kLeafRef || (nodes.size() + b.size()) * 4u > 0xffffff00ull)
+            return false;
+        // the BLAS trees move behind the TLAS's, and BLAS leaves behind the TLAS nodes
+        const uint32_t node_shift = static_cast<uint32_t>(nodes.size() / 4u);
+        const uint32_t leaf_shift = static_cast<uint32_t>(t.size());
+        auto move = [&](uint32_t &ref) { ref += (ref & kLeafRef) ? leaf_shift : node_shift; };
+        for (size_t at = 0; at < b.size(); at += 4u * units()) {
+            move(b[at + left_at()]);
+            move(b[at + right_at()]);
+        }
+        for (size_t i = d->tlas_nodes_len; i < t.size(); i++) move(t[i].left_or_custom_id);  // mesh leaves' copies
+        nodes.insert(nodes.end(), b.begin(), b.end());
         tlas = std::move(t);
-        blas = std::move(b);
         return true;
     }
 
@@ -1669,28 +1686,66 @@ private:
         }
     }
 
-    static bool grow(std::vector<orn_sah::Leaf> &leaves, std::vector<orn_bvh_node> &nodes, uint32_t *root)
+    // A node's 16-byte units and where its references are, in words.
+    uint32_t units() const { return format_ == 2u ? sizeof(SearchNode) / 16u : sizeof(orn_bvh_node) / 16u; }
+    uint32_t left_at() const
+    {
+        return (format_ == 2u ? offsetof(SearchNode, left) : offsetof(orn_bvh_node, left_or_custom_id)) / 4u;
+    }
+    uint32_t right_at() const
+    {
+        return (format_ == 2u ? offsetof(SearchNode, right) : offsetof(orn_bvh_node, right_or_material_index)) / 4u;
+    }
+
+    bool grow(std::vector<orn_sah::Leaf> &leaves, std::vector<uint32_t> &out, uint32_t *root) const
     {
         if (leaves.size() == 1) {
             *root = leaves[0].ref;
             return true;
         }
-        const size_t base = nodes.size();
-        if (base + leaves.size() >= kLeafRef) return false;
-        nodes.resize(base + leaves.size() - 1);
-        *root = static_cast<uint32_t>(base);
-        return orn_sah::Builder(leaves, nodes.data() + base, *root)
-            .build(orn_sah::ceil_log2(leaves.size()) + kExtraHeight,
-                   std::min(8u, std::max(1u, std::thread::hardware_concurrency())));
+        const size_t base = out.size() / (4u * units());
+        if ((base + leaves.size()) * units() >= kLeafRef) return false;
+        std::vector<orn_bvh_node> built(leaves.size() - 1);
+        if (!orn_sah::Builder(leaves, built.data(), static_cast<uint32_t>(base))
+                 .build(orn_sah::ceil_log2(leaves.size()) + kExtraHeight,
+                        std::min(8u, std::max(1u, std::thread::hardware_concurrency()))))
+            return false;
+        auto place = [&](uint32_t ref) { return (ref & kLeafRef) ? ref : ref * units(); };
+        out.reserve(out.size() + built.size() * 4u * units());
+        auto append = [&](const void *node) {
+            const uint32_t *w = static_cast<const uint32_t *>(node);
+            out.insert(out.end(), w, w + 4u * units());
+        };
+        for (orn_bvh_node &n : built) {
+            n.left_or_custom_id = place(n.left_or_custom_id);
+            n.right_or_material_index = place(n.right_or_material_index);
+            if (format_ != 2u) {
+                append(&n);
+                continue;
+            }
+            SearchNode s;
+            for (int a = 0; a < 3; a++) {
+                const float p[6] = {n.lmin_or_v0[a], n.rmin_or_v2[a], n.lmax_or_v1[a],
+                                    n.rmax_or_v3[a], n.lmin_or_v0[a], n.rmin_or_v2[a]};
+                std::memcpy(s.plane[a], p, sizeof(p));
+            }
+            s.left = n.left_or_custom_id;
+            s.right = n.right_or_material_index;
+            append(&s);
+        }
+        *root = place(static_cast<uint32_t>(base));
+        return true;
     }
 
     // Stack entries a traversal from `ref` on needs whichever child it takes first.
-    static uint32_t pending(const std::vector<orn_bvh_node> &n, uint32_t ref, const std::vector<uint32_t> *below)
+    uint32_t pending(const std::vector<uint32_t> &n, uint32_t ref, const std::vector<uint32_t> *below) const
     {
         if (ref & kLeafRef) return below ? (*below)[ref & ~kLeafRef] : 0u;
-        return 1u + std::max(pending(n, n[ref].left_or_custom_id, below),
-                             pending(n, n[ref].right_or_material_index, below));
+        const size_t at = size_t{ref} * 4u;
+        return 1u + std::max(pending(n, n[at + left_at()], below), pending(n, n[at + right_at()], below));
     }
+
+    uint32_t format_;
 };
 
 // Uploads validated arrays. `roots` are the TLAS root indices of the scenes
@@ -1773,15 +1828,15 @@ orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots
         ds.tlas2_root = root2[0];
         ds.plain_spheres = spheres_are_plain(desc) ? 1u : 0u;
         if (ds.plain_spheres) fill_sphere_leaves(desc, t2);
-        SearchTree search;
+        SearchTree search(bvh2_format(s->features));
         bool ordered = false;
         try {
-            ordered = search.build(desc, roots, n_roots, t2, b2);
+            ordered = search.build(desc, roots, n_roots, t2);
         } catch (...) {  // no memory for it: the reference's order throughout
         }
         for (size_t i = 0; i < n_roots; i++) search_root[i] = ordered ? search.roots[i] : root2[i];
         ds.search_root = search_root[0];
-        ds.ordered = ordered ? 1u : 0u;
+        if (!ordered) s->features |= kNoSearchTree;
         s->traversal_slots = ordered ? std::max(slots, search.slots) : slots;
         float size = 0.0f;  // largest coordinate of the scene
         for (int a = 0; a < 3; a++)
@@ -1792,17 +1847,22 @@ orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots
         const size_t tlas_n = t2.size();
         if (tlas_n + b2.size() >= kLeafRef) return fail(ORN_ERROR_OUT_OF_MEMORY);
         const uint32_t shift = static_cast<uint32_t>(tlas_n);  // leaves the flag alone
-        for (orn_bvh_node &nd : t2)
-            if (nd.node_type == 2u) nd.left_or_custom_id += shift;
+        for (size_t i = 0; i < desc->tlas_nodes_len; i++)  // (the search tree's copies have their own roots)
+            if (t2[i].node_type == 2u) t2[i].left_or_custom_id += shift;
         for (orn_bvh_node &nd : b2)
             if (nd.node_type == 0u) {
                 nd.left_or_custom_id += shift;
                 nd.right_or_material_index += shift;
             }
         t2.insert(t2.end(), b2.begin(), b2.end());
+        // and the search tree in front of it (one allocation: the two are read in turn)
+        const size_t ahead = ordered ? (search.nodes.size() + 15) / 16 : 0;
+        t2.insert(t2.begin(), ahead, orn_bvh_node{});
+        if (ordered) std::memcpy(t2.data(), search.nodes.data(), 4 * search.nodes.size());
         if ((st = upload(s, reinterpret_cast<const float4 *>(t2.data()), 4 * t2.size(), &f4))) return fail(st);
-        ds.nodes2 = f4;
-        ds.blas2 = f4 + 4 * tlas_n;
+        ds.search = ordered ? reinterpret_cast<const char *>(f4) : nullptr;
+        ds.nodes2 = f4 + 4 * ahead;
+        ds.blas2 = ds.nodes2 + 4 * tlas_n;
     }
     // derived BVH4 arrays and the TLAS copy whose mesh leaves point at
     // their BLAS's BVH4 root
@@ -2262,7 +2322,9 @@ static orn_status trace_rays(orn_device_scene *s, float t_min, const float *rays
         const uint32_t c = static_cast<uint32_t>(count), blocks = blocks_for(c, kBlock);
         if (packet) trace_packet_kernel<<<blocks, kBlock, 0, st>>>(ds, t_min, d_rays, c, d_out);
         else if (s->trace_width == 4u) trace_kernel<4><<<blocks, kBlock, lds, st>>>(ds, t_min, d_rays, c, d_out);
-        else trace_kernel<2><<<blocks, kBlock, lds, st>>>(ds, t_min, d_rays, c, d_out);
+        else if (!ds.search) trace_kernel<1><<<blocks, kBlock, lds, st>>>(ds, t_min, d_rays, c, d_out);
+        else if (bvh2_format(s->features) == 2u) trace_kernel<2><<<blocks, kBlock, lds, st>>>(ds, t_min, d_rays, c, d_out);
+        else trace_kernel<3><<<blocks, kBlock, lds, st>>>(ds, t_min, d_rays, c, d_out);
         return hipGetLastError();
     };
     constexpr size_t kRay = 6 * sizeof(float);
@@ -2994,7 +3056,7 @@ std::string scene_class(const orn_device_scene *s, uint64_t pixels, uint32_t spp
 {
     char key[256];
     std::snprintf(key, sizeof(key), "%s|features%u|tlas2^%u|blas2^%u|px2^%u|spp2^%u|depth%u|images2^%u|bvh4%u",
-                  s->ctx->arch, s->features, log2_bucket(s->ds.tlas_len), log2_bucket(s->blas_len),
+                  s->ctx->arch, s->features & 7u, log2_bucket(s->ds.tlas_len), log2_bucket(s->blas_len),
                   log2_bucket(pixels), log2_bucket(std::max(spp, 1u)), depth, log2_bucket(images),
                   (flags & ORN_TUNE_ALLOW_BVH4) ? 1u : 0u);
     return key;

@@ -62,14 +62,33 @@ struct DevScene {
     uint32_t stack_slots;  // LDS stack entries per lane
     uint32_t tlas4_root;   // reference of the TLAS root in the BVH4
     uint32_t tlas2_root;   // index of the TLAS root, kLeafRef set when it is a leaf
-    // The search tree over the same leaves (orn_sah.h), kept behind the TLAS's
-    // and the BLASes' own nodes in nodes2; `ordered` 0: there is none, search_root is
-    // tlas2_root and rays take the reference's order throughout.
-    uint32_t search_root;
-    uint32_t ordered;
+    // The internal nodes of the search tree over the same leaves (orn_sah.h), in
+    // the format of bvh2_format(); null: there is none, and rays take the
+    // reference's order.
+    const char *__restrict__ search;
+    uint32_t search_root;  // as the search tree's references go
+    uint32_t pad;
     float cull_rel, cull_abs;  // slack of the ordered search's distance cull (trav_cull)
     uint32_t plain_spheres;    // every sphere is scaled along the axes and moved (see sphere_leaf)
 };
+
+// An internal node of the search tree of a scene without meshes: per axis the
+// children's planes as left min, right min, left max, right max, left min,
+// right min, so that one 16-byte load at an offset of 0 or 8, by the sign of
+// the ray's direction, gives both near planes and then both far planes: 12
+// minima and maxima of a node visit less. (The nearer of fma(min, inv, ox) and
+// fma(max, inv, ox) is the min plane's for inv > 0 and the max plane's for
+// inv < 0, whatever the rounding: fma is monotone.)
+// References of a search tree: a leaf's index in nodes2 with kLeafRef, or an
+// internal node's place in units of 16 bytes.
+struct alignas(8) SearchQuad {
+    float a, b, c, d;
+};
+struct SearchNode {
+    float plane[3][6];
+    uint32_t left, right;
+};
+static_assert(sizeof(SearchNode) == 80, "a search node is five 16-byte units");
 
 struct Hit {
     float t;
@@ -232,17 +251,27 @@ enum SceneFeatures : uint32_t {
     kHasSpheres = 1u,
     kHasMeshes = 2u,
     kHasTextures = 4u,
+    kNoSearchTree = 8u,  // BVH2 launches take the reference's order
 };
+// Node format of a BVH2 launch (the W of the traversal below). The wider nodes
+// of format 2 take a quarter more of the caches for their shorter test: random
+// spheres 1920x1080, 64 spp, 23.8 -> 23.3 ms with them and 500x500, 1 spp, 0.25 ->
+// 0.235 ms, but 1,024 instanced icospheres 20.4 -> 20.9 ms (cost-ordered, 32 spp; a
+// stride of 96 bytes 21.1, of 128 bytes 22.1). So the trees of a mesh scene,
+// which are the large ones, keep the 64-byte boxes.
+constexpr uint32_t bvh2_format(uint32_t f) { return (f & kNoSearchTree) ? 1u : (f & kHasMeshes) ? 3u : 2u; }
+constexpr bool is_search_format(uint32_t w) { return w == 2u || w == 3u; }
 
 // bvh.wgsl:14-137 as a resumable state machine: trav_begin() sets up one ray,
 // trav_internal()/trav_leaf() visit one node and return false once the ray is
 // finished. The node taken next is kept in a register: only nodes left for
 // later go to the lane's LDS column (`stack`, stride = block size).
 //
-// Two searches share the code. With ORD = false the order is the reference's
-// (left pushed before right, so the right child is taken first), with the
-// same strict `t < t_max` update. With ORD = true (BVH2 launches) the ray
-// searches the scene's SAH tree, the nearer child first, and finds the same
+// The searches share the code, by the node format W. With W = 1 the order is
+// the reference's (left pushed before right, so the right child is taken
+// first), with the same strict `t < t_max` update; W = 4 is the BVH4 below.
+// With W = 2 (SearchNode) and W = 3 (the BVH2's own node) the ray searches
+// the scene's SAH tree, the nearer child first, and finds the same
 // closest hit with far fewer node visits:
 //  * A primitive is in reach of a ray when the ray passes the slab test of
 //    its own leaf box without a distance limit. Every box above contains that
@@ -264,24 +293,32 @@ enum SceneFeatures : uint32_t {
 // visits are time: random spheres 1920x1080, 64 spp, 52 -> 33 ms; 1,024
 // instanced icospheres, 32 spp, 40 -> 30 ms; a batch of 16 instanced scenes
 // 25 -> 15 ms (with the same launch shapes, readback included). Scenes whose
-// arrays do not have nested boxes (SearchTree::build) keep ORD's order equal
-// to the reference's (sc.ordered 0).
+// arrays do not have nested boxes (SearchTree::build) have no search tree.
 struct Traversal {
     Ray ray;        // the ray in object space, inside a BLAS
     f3 inv, ox;     // safe_invdir(d) and -o * inv of the ray in the current space
     f3 winv, wox;   // the same of the world-space ray, restored on leaving a BLAS
+    uint32_t sx, sy, sz;  // W = 2: plane offsets of a SearchNode by the signs of inv
     float t_max;
-    float t_cull;     // ORD: boxes and hits beyond it are skipped
-    float mesh_near;  // ORD: where the ray enters the box of the instance it is in
+    float t_cull;     // search tree: boxes and hits beyond it are skipped
+    float mesh_near;  // search tree: where the ray enters the box of the instance it is in
     uint32_t addr;  // next node to visit
     uint32_t top;   // pending entries in the LDS column
     uint32_t material_index, inv_tid;  // of the mesh being traversed
     uint32_t blas_top;  // `top` when the ray entered the BLAS it is in (kInTlas: none)
     bool hit;
-    bool early;  // ORD: the closest hit lies in front of its own box
-    bool redo;   // ORD: the closest hit needs the reference's order (see above)
+    bool early;  // search tree: the closest hit lies in front of its own box
+    bool redo;   // search tree: the closest hit needs the reference's order (see above)
     Hit h;
 };
+
+// Where a ray finds its near planes in a SearchNode's three axes.
+__device__ __forceinline__ void trav_signs(Traversal &tr)
+{
+    tr.sx = (as_u32(tr.inv.x) >> 31) * 8u;
+    tr.sy = (as_u32(tr.inv.y) >> 31) * 8u + 24u;
+    tr.sz = (as_u32(tr.inv.z) >> 31) * 8u + 48u;
+}
 
 // `root`: the TLAS root reference in the traversed format (BVH2, its search
 // tree, or BVH4).
@@ -289,6 +326,7 @@ __device__ __forceinline__ void trav_begin(uint32_t root, const Ray &world, Trav
 {
     tr.inv = safe_invdir(world.d);
     tr.ox = (-world.o) * tr.inv;
+    trav_signs(tr);
     tr.winv = tr.inv;
     tr.wox = tr.ox;
     tr.t_max = kTMaxInit;
@@ -315,7 +353,7 @@ __device__ __forceinline__ void pin_node(float4 &a, float4 &b, float4 &c, float4
 // Takes the next pending node off the lane's stack; false when none is left.
 // A BLAS is done when the stack is down to where it was on entering it (the
 // reference pushes a marker instead, bvh.wgsl:88-95).
-template <uint32_t F>
+template <uint32_t F, uint32_t W>
 __device__ __forceinline__ bool trav_pop(uint32_t *stack, uint32_t stride, Traversal &tr)
 {
     if (tr.top == 0u) return false;
@@ -375,21 +413,20 @@ __device__ __forceinline__ bool bvh4_node(const float4 *nd, uint32_t *stack, uin
 template <uint32_t F>
 __device__ __forceinline__ void trav_cull(const DevScene &sc, Traversal &tr, float t, float t_old, float near_t)
 {
-    const bool ordered = sc.ordered != 0u;
     const f3 wi = (F & kHasMeshes) ? tr.winv : tr.inv;
     const float inv = fmaxf(fmaxf(fabsf(wi.x), fabsf(wi.y)), fabsf(wi.z));
     float off = fmaxf(fmaxf(fabsf(tr.ox.x), fabsf(tr.ox.y)), fabsf(tr.ox.z));
     if (F & kHasMeshes) off = fmaxf(off, fmaxf(fmaxf(fabsf(tr.wox.x), fabsf(tr.wox.y)), fabsf(tr.wox.z)));
     const float slack = fmaf(sc.cull_rel, fabsf(t), fmaf(sc.cull_abs, inv, kCullUlp * off));
-    tr.t_cull = ordered ? fmaxf(t, near_t) + slack : t;
-    tr.early = ordered && near_t > t;
-    tr.redo = ordered && near_t > t_old;
+    tr.t_cull = fmaxf(t, near_t) + slack;
+    tr.early = near_t > t;
+    tr.redo = near_t > t_old;
 }
 
 // A hit at t no closer than the best one, but not beyond t_cull.
-__device__ __forceinline__ void trav_behind(const DevScene &sc, Traversal &tr, float t)
+__device__ __forceinline__ void trav_behind(Traversal &tr, float t)
 {
-    if (sc.ordered != 0u && (tr.early || t == tr.t_max)) tr.redo = true;
+    if (tr.early || t == tr.t_max) tr.redo = true;
 }
 
 // Node references carry kLeafRef when they name a leaf (in the BVH4 by
@@ -397,7 +434,7 @@ __device__ __forceinline__ void trav_behind(const DevScene &sc, Traversal &tr, f
 // whether its next step is an internal node or a leaf before loading it.
 // trav_internal() visits an internal node, trav_leaf() a leaf; both return
 // false once the ray is finished.
-template <uint32_t F, uint32_t W, bool ORD>
+template <uint32_t F, uint32_t W>
 __device__ __forceinline__ bool trav_internal(const DevScene &sc, float t_min, const Ray &world,
                                               uint32_t *stack, uint32_t stride, Traversal &tr)
 {
@@ -406,33 +443,57 @@ __device__ __forceinline__ bool trav_internal(const DevScene &sc, float t_min, c
         const bool blas = (F & kHasMeshes) && tr.blas_top != kInTlas;
         const float4 *nd = (blas ? sc.blas4 : sc.tlas4) + 8u * tr.addr;
         if (bvh4_node(nd, stack, stride, cap, t_min, tr)) return true;
-        return trav_pop<F>(stack, stride, tr);
+        return trav_pop<F, W>(stack, stride, tr);
     }
-    const float4 *node = sc.nodes2 + 4u * tr.addr;
-    float4 n0 = node[0], n1 = node[1], n2 = node[2], n3 = node[3];
-    const float limit = ORD ? tr.t_cull : tr.t_max;
-    float ln, rn;
-    const bool l = aabb_hit(make_float3(n0.x, n0.y, n0.z), make_float3(n1.x, n1.y, n1.z), tr.inv,
-                            tr.ox, t_min, limit, ln);
-    const bool r = aabb_hit(make_float3(n2.x, n2.y, n2.z), make_float3(n3.x, n3.y, n3.z), tr.inv,
-                            tr.ox, t_min, limit, rn);
-    // both hit: one child is next, the other waits on the stack (in the
-    // reference's order the left one)
-    const bool left_first = !r | (ORD & (sc.ordered != 0u) & l & (ln < rn));
-    if (l && r && tr.top < cap) stack[(tr.top++) * stride] = left_first ? as_u32(n1.w) : as_u32(n0.w);
+    bool l, r;
+    uint32_t left, right;
+    bool left_first;
+    if constexpr (W == 2u) {
+        const uint32_t off = tr.addr << 4;  // 32 bits from a scalar base: the tree is at most 4 GB
+        auto quad = [&](uint32_t o) { return *reinterpret_cast<const SearchQuad *>(sc.search + (off + o)); };
+        const SearchQuad x = quad(tr.sx), y = quad(tr.sy), z = quad(tr.sz);
+        const uint2 kids = *reinterpret_cast<const uint2 *>(sc.search + off + offsetof(SearchNode, left));
+        left = kids.x;
+        right = kids.y;
+        const float ln = fmaxf(fmaxf(fmaxf(fmaf(x.a, tr.inv.x, tr.ox.x), fmaf(y.a, tr.inv.y, tr.ox.y)),
+                                     fmaf(z.a, tr.inv.z, tr.ox.z)), t_min);
+        const float rn = fmaxf(fmaxf(fmaxf(fmaf(x.b, tr.inv.x, tr.ox.x), fmaf(y.b, tr.inv.y, tr.ox.y)),
+                                     fmaf(z.b, tr.inv.z, tr.ox.z)), t_min);
+        const float lf = fminf(fminf(fminf(fmaf(x.c, tr.inv.x, tr.ox.x), fmaf(y.c, tr.inv.y, tr.ox.y)),
+                                     fmaf(z.c, tr.inv.z, tr.ox.z)), tr.t_cull);
+        const float rf = fminf(fminf(fminf(fmaf(x.d, tr.inv.x, tr.ox.x), fmaf(y.d, tr.inv.y, tr.ox.y)),
+                                     fmaf(z.d, tr.inv.z, tr.ox.z)), tr.t_cull);
+        l = ln <= lf;
+        r = rn <= rf;
+        left_first = !r | (l & (ln < rn));  // the nearer child
+    } else {
+        constexpr bool ORD = W == 3u;
+        const float4 *node = ORD ? reinterpret_cast<const float4 *>(sc.search + (tr.addr << 4)) : sc.nodes2 + 4u * tr.addr;
+        const float4 n0 = node[0], n1 = node[1], n2 = node[2], n3 = node[3];
+        const float limit = ORD ? tr.t_cull : tr.t_max;
+        float ln, rn;
+        l = aabb_hit(make_float3(n0.x, n0.y, n0.z), make_float3(n1.x, n1.y, n1.z), tr.inv, tr.ox, t_min, limit, ln);
+        r = aabb_hit(make_float3(n2.x, n2.y, n2.z), make_float3(n3.x, n3.y, n3.z), tr.inv, tr.ox, t_min, limit, rn);
+        left = as_u32(n0.w);
+        right = as_u32(n1.w);
+        left_first = !r | (ORD & l & (ln < rn));  // the nearer child, or the reference's order: right first
+    }
+    // both hit: one child is next, the other waits on the stack
+    if (l && r && tr.top < cap) stack[(tr.top++) * stride] = left_first ? right : left;
     if (l || r) {
-        tr.addr = left_first ? as_u32(n0.w) : as_u32(n1.w);
+        tr.addr = left_first ? left : right;
         return true;
     }
-    return trav_pop<F>(stack, stride, tr);
+    return trav_pop<F, W>(stack, stride, tr);
 }
 
-template <uint32_t F, uint32_t W, bool ORD>
+template <uint32_t F, uint32_t W>
 __device__ __forceinline__ bool trav_leaf(const DevScene &sc, float t_min, const Ray &world,
                                           uint32_t *stack, uint32_t stride, Traversal &tr)
 {
     const uint32_t idx = tr.addr & ~kLeafRef;
-    const float4 *base = W == 2u ? sc.nodes2 : ((F & kHasMeshes) && tr.blas_top != kInTlas ? sc.blas2 : sc.tlas_leaves);
+    constexpr bool ORD = is_search_format(W);
+    const float4 *base = W != 4u ? sc.nodes2 : ((F & kHasMeshes) && tr.blas_top != kInTlas ? sc.blas2 : sc.tlas_leaves);
     const float4 *node = base + 4u * idx;
     float4 n0 = node[0], n1 = node[1], n2 = node[2], n3 = node[3];
     // Keep the four 16-byte loads of the node together ahead of the type
@@ -460,7 +521,7 @@ __device__ __forceinline__ bool trav_leaf(const DevScene &sc, float t_min, const
                 trav_cull<F>(sc, tr, t, t_old, near_t);
             }
         } else if (ORD && ok) {
-            trav_behind(sc, tr, t);
+            trav_behind(tr, t);
         }
     } else if ((F & kHasMeshes) && type == 2u) {
         if constexpr (ORD)
@@ -499,10 +560,10 @@ __device__ __forceinline__ bool trav_leaf(const DevScene &sc, float t_min, const
                 trav_cull<F>(sc, tr, t, t_old, fmaxf(near_t, tr.mesh_near));
             }
         } else if (ORD && ok) {
-            trav_behind(sc, tr, t);
+            trav_behind(tr, t);
         }
     }
-    return trav_pop<F>(stack, stride, tr);
+    return trav_pop<F, W>(stack, stride, tr);
 }
 
 // The ray of a finished ordered search once more, in the reference's order
@@ -513,8 +574,8 @@ __device__ __forceinline__ void trav_redo(const DevScene &sc, uint32_t root, flo
 {
     trav_begin(root, world, tr);
     for (bool on = true; on;)
-        on = (tr.addr & kLeafRef) ? trav_leaf<F, 2, false>(sc, t_min, world, stack, stride, tr)
-                                  : trav_internal<F, 2, false>(sc, t_min, world, stack, stride, tr);
+        on = (tr.addr & kLeafRef) ? trav_leaf<F, 1>(sc, t_min, world, stack, stride, tr)
+                                  : trav_internal<F, 1>(sc, t_min, world, stack, stride, tr);
 }
 
 // The whole of bvh_hit for one ray. With STEPS > 1 a lane visits up to STEPS
@@ -526,14 +587,14 @@ template <uint32_t F, uint32_t W, uint32_t STEPS = 1>
 __device__ __forceinline__ bool bvh_hit(const DevScene &sc, float t_min, const Ray &world,
                                         uint32_t *stack, uint32_t stride, Hit &h)
 {
-    constexpr bool ORD = W == 2u;
+    constexpr bool ORD = is_search_format(W);
     Traversal tr;
-    trav_begin(W == 4u ? sc.tlas4_root : sc.search_root, world, tr);
+    trav_begin(W == 4u ? sc.tlas4_root : ORD ? sc.search_root : sc.tlas2_root, world, tr);
     bool on = true;
     while (on) {
         for (uint32_t k = 0; k < STEPS && on && !(tr.addr & kLeafRef); k++)
-            on = trav_internal<F, W, ORD>(sc, t_min, world, stack, stride, tr);
-        if (on && (tr.addr & kLeafRef)) on = trav_leaf<F, W, ORD>(sc, t_min, world, stack, stride, tr);
+            on = trav_internal<F, W>(sc, t_min, world, stack, stride, tr);
+        if (on && (tr.addr & kLeafRef)) on = trav_leaf<F, W>(sc, t_min, world, stack, stride, tr);
     }
     if (ORD && tr.redo) trav_redo<F>(sc, sc.tlas2_root, t_min, world, stack, stride, tr);
     h = tr.h;
