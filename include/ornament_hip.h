@@ -316,7 +316,8 @@ orn_status orn_get_accumulation(orn_target *target, float *dst, size_t pixels);
 orn_status orn_get_rng_state(orn_target *target, uint32_t *dst, size_t pixels);
 /* Per-pixel cost recorded by the target's latest render with tuning
  * cost_order 1: the GPU time of the pixel's jobs, in ticks of the 100 MHz
- * device clock (width * height entries, row-major like the accumulation).
+ * device clock (width * height entries, row-major like the accumulation);
+ * time in a wave that held back most of its lanes for the pixel counts twice.
  * No counterpart in the reference; it is what orders the next render's
  * queues. ORN_ERROR_INVALID_VALUE if no render has recorded costs. */
 orn_status orn_get_pixel_costs(orn_target *target, uint32_t *dst, size_t pixels);

@@ -55,9 +55,14 @@ constexpr uint32_t kQueueStride = 32;
 // end (a quarter instead of a 64th: a 16-image batch 12.4 -> 15 ms). Only for
 // whole pixels: a wave must not hold a split pixel's job back while all its
 // lanes wait for jobs that other waves hold back.
+constexpr uint32_t kAheadShare = 64, kAheadMost = 64;
 // Most lanes of a sparse wave, and the step they come in (launch_render_k).
 constexpr uint32_t kSparseLanes = 8, kLaneStep = 4;
-constexpr uint32_t kAheadShare = 64, kAheadMost = 64;
+// Heavy pixels (start_queues_kernel): lanes of a wave that takes them, at most
+// one wave in kHeavyShare, those above kHeavyPart of the costliest pixel, and
+// what a heavy wave's time stands for in a full wave.
+constexpr uint32_t kHeavyLanes = 4, kHeavyShare = 4, kHeavyScale = 2;
+constexpr float kHeavyPart = 0.5f;
 constexpr uint32_t kQueueWords = kXcds * kQueueStride;
 constexpr uint32_t kMaxStack = 63;  // the reference's private stack has 64 slots
 constexpr uint64_t kMaxPixels = 1ull << 28;  // per target or batch: 4 GiB of accumulation
@@ -78,6 +83,7 @@ struct KernelParams {
     uint32_t split_pct;     // percentage of each band's pixels that are split
     uint32_t pixels;        // pixels in the pixel buffers (at most 2^28)
     uint32_t lanes;         // lanes of each wave that take pixels (the rest stay idle)
+    uint32_t heavy;         // the queues start with heavy pixels (start_queues_kernel)
     const uint32_t *order;  // queue position -> tile-pixel of the band, or null: tile order
     uint32_t *cost;         // per-pixel job time to record, or null
 };
@@ -180,7 +186,9 @@ __device__ __forceinline__ void store_coherent(__amdgpu_buffer_rsrc_t r, uint32_
 // With a queue order (tuning cost_order), position q of a band's queue is
 // the band's tile-pixel order[q] instead of the q-th: the pixels that cost
 // most in the previous render come first, so the jobs drawn last are cheap
-// and the lanes run out of work nearly together.
+// and the lanes run out of work nearly together. The costliest of them may be
+// heavy pixels (start_queues_kernel): those belong to the band's first waves,
+// which give all but a few lanes nothing until they are done.
 // Within a wave, a lane alternates between traversing its current ray one
 // node per loop iteration and a shading round (hit shading, accumulation,
 // next camera path, next job). A lane whose traversal ended waits; the wave
@@ -281,6 +289,23 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
     Traversal tr;
     tr.addr = kLeafRef;  // a lane that is not traversing holds a leaf-flagged reference
     tr.redo = false;
+    // Jobs [held_at, held_at + held) of the band are the wave's, drawn but not
+    // yet given to lanes; its next draw takes `ahead` more than lanes ask for.
+    uint32_t held_at = 0, held = 0, ahead = 0;
+    // A heavy wave (wave-uniform) starts with up to kHeavyLanes heavy pixels and
+    // draws nothing more until they are done. The band's waves are counted so
+    // that neighbours sit in different workgroups and on different SIMDs.
+    bool heavy = false;
+    if (kp.heavy) {
+        const uint32_t blocks = gridDim.x / kXcds, b = blockIdx.x / kXcds;
+        const uint32_t k = (threadIdx.x / 64u + b) % (kBlock / 64u) * blocks + b;
+        const uint32_t n = __builtin_amdgcn_readfirstlane(queues[blockIdx.x % kXcds * kQueueStride + 1u]);
+        held_at = __builtin_amdgcn_readfirstlane(k * kHeavyLanes);
+        if (held_at < n) {
+            heavy = true;
+            held = min(kHeavyLanes, n - held_at);
+        }
+    }
     uint32_t mode = lane < kp.lanes ? kWaiting : kDone;
     bool need_pixel = true;
     bool blocked = false;  // holds a job whose predecessor has not finished
@@ -326,8 +351,8 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
     auto end_job = [&]() {
         uint32_t *cost = reload_args().kp.cost;
         if (cost)  // the pixel's cost for the next render's queue order
-            __hip_atomic_fetch_add(cost + pix, device_ticks() - job_t0, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(cost + pix, (device_ticks() - job_t0) * (heavy ? kHeavyScale : 1u),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (job + 1u < lane_chunks) {  // handed on; released at the wave's next flush
             store_coherent(acc_rsrc, pix, acc);
             store_coherent(rng_buf + pix, rng);
@@ -428,14 +453,11 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
 
     uint32_t band = blockIdx.x % kXcds;  // wave-uniform
     uint32_t bands_left = kXcds - 1u;    // bands to visit after this one
-    // Jobs [held_at, held_at + held) of the band are the wave's, drawn but not
-    // yet given to lanes; its next draw takes `ahead` more than lanes ask for.
-    uint32_t held_at = 0, held = 0, ahead = 0;
     uint32_t band_px = band_pixels(band);
     uint32_t band_split = split_pixels(band_px);
     uint32_t band_jobs = band_px - band_split + band_split * max_chunks();
     const uint32_t regroup = kp.regroup;
-    const uint32_t leaf_regroup = kp.leaf_regroup;
+    uint32_t leaf_regroup = heavy ? 1u : kp.leaf_regroup;
     const uint32_t node_steps = kp.node_steps;
     bool shade_all = false;  // POOL: this iteration's workgroup-wide shading decision
     for (;;) {
@@ -615,6 +637,14 @@ __global__ __launch_bounds__(kBlock, POOL ? 3 : 4) void render_kernel(DevScene s
             const int leader = __ffsll(static_cast<unsigned long long>(needy)) - 1;
             const uint32_t count = static_cast<uint32_t>(__popcll(needy));
             if (held == 0u) {
+                if (heavy) {
+                    // (idle lanes count as waiting, so a heavy wave comes here
+                    // after every run of node steps: a heavy pixel never waits
+                    // for a shading round)
+                    if (lanes_where(mode == kTraverse || (mode == kWaiting && !need_pixel)) != 0u) break;
+                    heavy = false;
+                    leaf_regroup = reload_args().kp.leaf_regroup;
+                }
                 held = count + ahead;
                 uint32_t base = 0;
                 if (lane == static_cast<uint32_t>(leader)) base = atomicAdd(queues + band * kQueueStride, held);
@@ -740,9 +770,49 @@ __global__ __launch_bounds__(kBlock) void post_batch_kernel(const BatchItem *__r
     if (x < it.p.width && y < it.p.height) post_pixel(it.p, it.count, x, y, acc + it.px_base, fb + it.px_base);
 }
 
-__global__ void reset_queues_kernel(uint32_t *q)
+// Starts the bands' queues. With `totals` (the pixels of each band and cost
+// class) it also counts each band's heavy pixels, into the counter's second
+// word; they are the first of the band's order and go to its first waves,
+// kHeavyLanes each (render_kernel). One wave per band.
+// Why: a pixel is one lane's work, so a launch takes at least the time of its
+// costliest one, and in a full wave every step of that pixel waits for 63
+// other lanes' node, leaf and shading rounds. Where that is what binds (1,024
+// instanced icospheres 1080p, 32 spp: the launch 20.6 ms, its costliest pixel
+// 20.5, all pixels spread evenly over the lanes 15), the few pixels above both
+// an even share and half of the costliest run at half the time in waves of 4:
+// 20.6 -> 18.4 ms; an instanced scene of 490,000 pixels, 8 spp 3.75 -> 3.37; 16
+// images of 630,000 pixels 9.5 (in tile order; ordered before 9.9) -> 6.45.
+// Random spheres 1080p, 64 spp, has no such pixels and keeps its 23.2. Waves of 2 to
+// 8 heavy lanes, shares of a half or a quarter and parts of 0.4 to 0.6 differ by less
+// than 2 %; 16 lanes cost 4 %, and no limit on the share 15 %.
+__global__ __launch_bounds__(64 * kXcds) void start_queues_kernel(uint32_t *q, const uint32_t *__restrict__ totals,
+                                                                  uint32_t lanes)
 {
-    if (threadIdx.x < kXcds) q[threadIdx.x * kQueueStride] = 0u;
+    const uint32_t band = threadIdx.x / 64u, lane = threadIdx.x % 64u;
+    uint32_t n = 0;
+    if (totals) {
+        float work = 0.0f, most = 0.0f;
+        for (uint32_t c = lane; c < kCostClasses; c += 64u) {
+            const float v = cost_of_class(c);
+            uint32_t all = 0;
+            for (uint32_t b = 0; b < kXcds; b++) all += totals[b * kCostClasses + c];
+            work += v * static_cast<float>(all);
+            if (all != 0u) most = fmaxf(most, v);
+        }
+        for (uint32_t d = 32; d != 0u; d >>= 1) {
+            work += __shfl_xor(work, d);
+            most = fmaxf(most, __shfl_xor(most, d));
+        }
+        const float limit = fmaxf(work / static_cast<float>(lanes), kHeavyPart * most);
+        for (uint32_t c = lane; c < kCostClasses; c += 64u)
+            if (cost_of_class(c) > limit) n += totals[band * kCostClasses + c];
+        for (uint32_t d = 32; d != 0u; d >>= 1) n += __shfl_xor(n, d);
+        n = min(n, lanes / (64u * kXcds * kHeavyShare) * kHeavyLanes);
+    }
+    if (lane == 0u) {
+        q[band * kQueueStride] = n;
+        q[band * kQueueStride + 1u] = n;
+    }
 }
 
 // Queue order by cost (tuning cost_order): a stable counting sort of each
@@ -1234,10 +1304,14 @@ orn_tuning default_tuning()
 // to 2 million pixels, 1 to 64 spp, as a geometric mean over 55 shapes): 7 %
 // less time than default_tuning(), 11 % with queues by cost. Those pay once
 // pixels are long (2000x1000, 15 spp 6.8 -> 6.35 ms; random spheres 1080p 64 spp
-// 29.9 -> 24.3; but 1080p 4 spp 2.49 -> 2.46, 500x500 1 spp 0.240 -> 0.258), or,
-// in a batch, once its images fill the lanes several times over (64 images of
-// 33 million pixels 140 -> 130 ms, 16 of 630,000 9.0 -> 9.9).
-constexpr uint32_t kCostOrderSpp = 8, kCostOrderBatchPixels = 1u << 21;
+// 29.9 -> 24.3; but 1080p 4 spp 2.49 -> 2.46, 500x500 1 spp 0.240 -> 0.258) and
+// many enough for the lanes to take more than one or for heavy pixels to have
+// lanes to spare (8 spp, plain -> ordered first -> later: instanced scenes 256x256
+// 1.87 -> 1.96 -> 1.91 ms, 512x512 2.22 -> 2.09 -> 1.99; Cornell boxes 0.77 -> 0.97
+// -> 0.81 and 1.20 -> 1.35 -> 1.11). A batch records its costs as it goes, so its
+// first render costs nothing more (131,072 to 1 million pixels of 1 to 32 spp: first
+// within 5 % of plain, later 5 to 30 % less; 32,768 pixels 1.15 -> 1.28).
+constexpr uint32_t kCostOrderSpp = 8, kCostOrderPixels = 1u << 17;
 orn_tuning untuned(bool cost_order)
 {
     orn_tuning t = default_tuning();
@@ -1320,6 +1394,7 @@ struct LaunchArgs {
     uint32_t *queues;
     uint32_t total_tiles;
     bool pool;  // tuning workgroup_pool (honoured for spheres-only scenes, BVH2, one image)
+    const uint32_t *totals = nullptr;  // of kp.order: pixels of each band and cost class
 };
 
 // One instantiation per combination of scene features.
@@ -1360,6 +1435,9 @@ hipError_t launch_render_k(uint32_t per_cu, uint32_t cus, size_t lds, hipStream_
         kp.regroup = std::max(1u, kp.regroup * kp.lanes / 64u);
         kp.leaf_regroup = std::max(1u, kp.leaf_regroup * kp.lanes / 64u);
     }
+    const bool whole = kp.split_pct == 0u || (!BATCH && kp.chunks == 1u);
+    kp.heavy = !POOL && kp.lanes == 64u && whole && a.totals ? 1u : 0u;
+    start_queues_kernel<<<1, 64 * kXcds, 0, st>>>(a.queues, kp.heavy ? a.totals : nullptr, grid * kBlock);
     render_kernel<F, W, BATCH, POOL>
         <<<grid, kBlock, lds, st>>>(ds, kp, a.items, a.work, a.acc, a.rng, a.stage, a.queues);
     return hipGetLastError();
@@ -2047,7 +2125,7 @@ namespace {
 hipError_t enqueue_render(orn_device_scene *s, const orn_constant_params *params, uint32_t iterations,
                           const orn_tuning &tuning, float4 *acc, uint32_t *rng, float4 *fb, uint32_t *stage,
                           uint32_t *queues, uint32_t epoch, hipStream_t st, const uint32_t *order = nullptr,
-                          uint32_t *cost = nullptr)
+                          uint32_t *cost = nullptr, const uint32_t *totals = nullptr)
 {
     KernelParams kp{};
     kp.p = *params;
@@ -2070,8 +2148,7 @@ hipError_t enqueue_render(orn_device_scene *s, const orn_constant_params *params
     kp.pixels = params->width * params->height;
     kp.order = order;
     kp.cost = cost;
-    LaunchArgs a{kp, nullptr, nullptr, acc, rng, stage, queues, kp.tiles, tuning.workgroup_pool != 0u};
-    reset_queues_kernel<<<1, 64, 0, st>>>(queues);
+    LaunchArgs a{kp, nullptr, nullptr, acc, rng, stage, queues, kp.tiles, tuning.workgroup_pool != 0u, totals};
     const hipError_t e = launch_render<false>(s->features, width, tuning.workgroups_per_cu,
                                               static_cast<uint32_t>(s->ctx->compute_units), lds, st, ds, a);
     if (e != hipSuccess || !fb) return e;
@@ -2138,7 +2215,7 @@ orn_status orn_render_async(orn_target *t, const orn_constant_params *params, ui
         }
     };
     next_epoch();
-    orn_tuning tuning = t->tuned ? t->tuning : untuned(iterations >= kCostOrderSpp);
+    orn_tuning tuning = t->tuned ? t->tuning : untuned(iterations >= kCostOrderSpp && n >= kCostOrderPixels);
     if (tuning.cost_order != 0u) {
         const hipError_t e = ensure_cost_order(t, st);
         if (e != hipSuccess && t->tuned) return from_hip(e);
@@ -2166,14 +2243,14 @@ orn_status orn_render_async(orn_target *t, const orn_constant_params *params, ui
         orn_constant_params rest = *params;
         rest.current_iteration = params->current_iteration + static_cast<float>(first);
         ORN_TRY(enqueue_render(s, &rest, iterations - first, tuning, t->acc, t->rng, t->fb, t->stage, t->queues,
-                               t->epoch, st, t->order, t->cost));
+                               t->epoch, st, t->order, t->cost, t->totals));
         ORN_TRY(hipEventRecord(t->ev_stop, st));
         t->timed = true;
         t->costs_recorded = true;
         return ORN_OK;
     }
     ORN_TRY(enqueue_render(s, params, iterations, tuning, t->acc, t->rng, t->fb, t->stage, t->queues, t->epoch,
-                           st, order, by_cost ? t->cost : nullptr));
+                           st, order, by_cost ? t->cost : nullptr, order ? t->totals : nullptr));
     ORN_TRY(hipEventRecord(t->ev_stop, st));
     t->timed = true;
     if (by_cost) t->costs_recorded = true;
@@ -2555,7 +2632,7 @@ struct orn_batch {
     uint32_t *queues;
     orn_tuning tuning;
     bool tuned = false;  // `tuning` was set; until then the library picks
-    orn_tuning launch_tuning() const { return tuned ? tuning : untuned(total_px >= kCostOrderBatchPixels); }
+    orn_tuning launch_tuning() const { return tuned ? tuning : untuned(total_px >= kCostOrderPixels); }
     hipGraph_t graph;
     hipGraphExec_t exec;
     bool graph_ok;
@@ -2657,7 +2734,15 @@ orn_status capture_batch(orn_batch *b)
     b->graph_ok = false;
     orn_device_scene *s = b->scene;
     hipStream_t st = s->ctx->stream;
-    const orn_tuning tuning = b->launch_tuning();
+    orn_tuning tuning = b->launch_tuning();
+    if (tuning.cost_order != 0u) {
+        const hipError_t e = ensure_batch_cost_order(b, st);
+        if (e != hipSuccess && b->tuned) return from_hip(e);
+        if (e != hipSuccess) {  // the order was not asked for
+            tuning.cost_order = 0u;
+            (void)hipGetLastError();
+        }
+    }
     const uint32_t width = tuning.bvh_width == 4u ? 4u : 2u;
     DevScene ds = s->ds;
     ds.stack_slots = width == 4u ? s->stack_slots4 : s->traversal_slots;
@@ -2670,11 +2755,10 @@ orn_status capture_batch(orn_batch *b)
     kp.pixels = b->total_px;
     const bool by_cost = tuning.cost_order != 0u;
     if (by_cost) {
-        ORN_TRY(ensure_batch_cost_order(b, st));
         kp.order = b->order;
         kp.cost = b->cost;
     }
-    LaunchArgs a{kp, b->d_items, b->d_work, b->acc, b->rng, b->stage, b->queues, b->total_tiles};
+    LaunchArgs a{kp, b->d_items, b->d_work, b->acc, b->rng, b->stage, b->queues, b->total_tiles, false, by_cost ? b->totals : nullptr};
     ORN_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
     hipError_t e = hipMemcpyAsync(b->d_items, b->h_items, b->n * sizeof(BatchItem), hipMemcpyHostToDevice, st);
     if (e == hipSuccess && by_cost) {
@@ -2682,10 +2766,6 @@ orn_status capture_batch(orn_batch *b)
         o.work = b->d_work;
         o.items = b->d_items;
         enqueue_order_kernels(o, b->total_tiles, b->cost, b->counts, b->totals, b->order, st);
-        e = hipGetLastError();
-    }
-    if (e == hipSuccess) {
-        reset_queues_kernel<<<1, 64, 0, st>>>(b->queues);
         e = hipGetLastError();
     }
     if (e == hipSuccess)

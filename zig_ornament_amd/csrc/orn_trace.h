@@ -1077,5 +1077,10 @@ __device__ __forceinline__ uint32_t cost_class(uint32_t c)
     const uint32_t f = e >= 2u ? (v >> (e - 2u)) & 3u : (v << (2u - e)) & 3u;
     return 4u * e + f;
 }
+// The least cost of a class.
+__device__ __forceinline__ float cost_of_class(uint32_t c)
+{
+    return ldexpf(1.0f + 0.25f * static_cast<float>(c & 3u), static_cast<int>(c >> 2)) - 1.0f;
+}
 
 }  // namespace orn
