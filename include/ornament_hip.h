@@ -268,7 +268,7 @@ orn_status orn_target_wait(orn_target *target);
  *   rest queued by them (two launches with the same result as one; a batch's
  *   first replay, or a render whose current_iteration is not a whole number
  *   below 2^24 - iterations, queues in tile order). orn_render_noalloc
- *   ignores it (default 0). */
+ *   takes the order from its own first samples (see there; default 0). */
 typedef struct orn_tuning {
     uint32_t regroup_lanes;
     uint32_t workgroups_per_cu;
@@ -291,11 +291,14 @@ orn_status orn_target_get_tuning(orn_target *target, orn_tuning *tuning);
  * `accumulation` (width * height float4, read and written), `rng`
  * (width * height uint32, read and written) and `framebuffer`
  * (width * height float4, written); width and height come from `params`.
- * The launch's scratch (the job-queue counters and one stage word per pixel
- * for split pixels) is a library-owned device array, one per device, sized
- * for ORN_RENDER_SCRATCH_PIXELS pixels (8 MiB) and held until the process
- * ends; larger images return ORN_ERROR_SCRATCH_TOO_SMALL before anything is
- * enqueued. `tuning` may be NULL (the library picks). `stream` is a
+ * The launch's scratch (the job-queue counters, one stage word per pixel for
+ * split pixels, and the buffers of cost_order) is a library-owned device
+ * array, one per device, sized for ORN_RENDER_SCRATCH_PIXELS pixels (30 MiB)
+ * and held until the process ends; larger images return
+ * ORN_ERROR_SCRATCH_TOO_SMALL before anything is enqueued. `tuning` may be
+ * NULL (the library picks); its cost_order applies from 8 samples and 131,072
+ * pixels on, if no pixel is split and the image has at most 9,216 tiles of
+ * 16x16, by the costs of the call's own first samples. `stream` is a
  * hipStream_t of the scene's device, or NULL for the device context's own
  * stream. The call returns once the work is enqueued. Every call on a device
  * uses the same scratch: calls whose work overlaps in time on one device (on

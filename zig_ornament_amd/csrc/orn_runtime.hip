@@ -1479,16 +1479,27 @@ hipError_t launch_render(uint32_t features, uint32_t width, uint32_t per_cu, uin
 
 }  // namespace
 
-// Scratch of orn_render_noalloc: the band queue counters, then one stage
-// word per pixel. Each device holds its own copy for the life of the
+// Scratch of orn_render_noalloc: the band queue counters, one stage word per
+// pixel, and what the queue order by cost takes (per pixel its cost, which is
+// zero between calls, the order of up to kScratchTiles tiles, and the class
+// counts). Each device holds its own copy for the life of the
 // process. Host code reaches it only through the address
 // hipGetSymbolAddress returns for the device (kept in g_scratch); the
 // array's name is not a device address on the host.
-constexpr uint32_t kScratchQueueWords = kQueueWords;
-static __device__ __align__(256) uint32_t scratch[kScratchQueueWords + ORN_RENDER_SCRATCH_PIXELS];
+constexpr uint32_t kScratchTiles = ORN_RENDER_SCRATCH_PIXELS / (kTile * kTile) / 8 * 9;  // a multiple of kXcds
+static_assert(kScratchTiles % kXcds == 0, "the bands' positions fit");
+struct Scratch {
+    uint32_t queues[kQueueWords];
+    uint32_t stage[ORN_RENDER_SCRATCH_PIXELS];
+    uint32_t cost[ORN_RENDER_SCRATCH_PIXELS];
+    uint32_t order[kScratchTiles * kTile * kTile];
+    uint32_t counts[kScratchTiles * kCostClasses];
+    uint32_t totals[kXcds * kCostClasses];
+};
+static __device__ __align__(256) Scratch scratch;
 
 struct ScratchSlot {
-    uint32_t *ptr;   // this device's scratch (device address)
+    Scratch *ptr;    // this device's scratch (device address)
     uint32_t epoch;  // tag of the latest orn_render_noalloc launch on the device
 };
 constexpr int kMaxDevices = 64;
@@ -1504,7 +1515,7 @@ static hipError_t init_scratch(int device)
     void *p = nullptr;
     const hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
     if (e != hipSuccess) return e;
-    g_scratch[device].ptr = static_cast<uint32_t *>(p);
+    g_scratch[device].ptr = static_cast<Scratch *>(p);
     g_scratch[device].epoch = 0;  // the array starts zeroed: no stage word carries a tag
     return hipSuccess;
 }
@@ -2182,17 +2193,18 @@ hipError_t ensure_cost_order(orn_target *t, hipStream_t st)
     return hipGetLastError();
 }
 
-// The queue order of a target's next render from the costs its previous
+// The queue order of an image's next render from the costs its previous
 // recording render left (and the costs cleared for the next recording).
-void enqueue_queue_order(orn_target *t, hipStream_t st)
+void enqueue_queue_order(uint32_t width, uint32_t height, uint32_t *cost, uint32_t *counts, uint32_t *totals,
+                         uint32_t *order, hipStream_t st)
 {
     OrderShape o{};
-    o.tiles_x = blocks_for(t->width, kTile);
-    o.tiles = o.tiles_x * blocks_for(t->height, kTile);
+    o.tiles_x = blocks_for(width, kTile);
+    o.tiles = o.tiles_x * blocks_for(height, kTile);
     o.tiles_per_xcd = blocks_for(o.tiles, kXcds);
-    o.width = t->width;
-    o.height = t->height;
-    enqueue_order_kernels(o, o.tiles, t->cost, t->counts, t->totals, t->order, st);
+    o.width = width;
+    o.height = height;
+    enqueue_order_kernels(o, o.tiles, cost, counts, totals, order, st);
 }
 
 }  // namespace
@@ -2228,7 +2240,7 @@ orn_status orn_render_async(orn_target *t, const orn_constant_params *params, ui
     ORN_TRY(hipEventRecord(t->ev_start, st));
     const uint32_t *order = nullptr;
     if (by_cost && t->costs_recorded) {
-        enqueue_queue_order(t, st);
+        enqueue_queue_order(t->width, t->height, t->cost, t->counts, t->totals, t->order, st);
         order = t->order;
     } else if (by_cost && splits_exactly(params->current_iteration, iterations) && iterations >= 2u) {
         // No costs recorded yet: the first eighth of the samples runs in
@@ -2239,7 +2251,7 @@ orn_status orn_render_async(orn_target *t, const orn_constant_params *params, ui
         ORN_TRY(enqueue_render(s, params, first, tuning, t->acc, t->rng, nullptr, t->stage, t->queues, t->epoch,
                                st, nullptr, t->cost));
         next_epoch();
-        enqueue_queue_order(t, st);
+        enqueue_queue_order(t->width, t->height, t->cost, t->counts, t->totals, t->order, st);
         orn_constant_params rest = *params;
         rest.current_iteration = params->current_iteration + static_cast<float>(first);
         ORN_TRY(enqueue_render(s, &rest, iterations - first, tuning, t->acc, t->rng, t->fb, t->stage, t->queues,
@@ -2266,6 +2278,7 @@ orn_status orn_render_noalloc(orn_device_scene *s, const orn_constant_params *pa
     if (params->width == 0 || params->height == 0) return ORN_ERROR_INVALID_VALUE;
     if (uint64_t(params->width) * params->height > ORN_RENDER_SCRATCH_PIXELS) return ORN_ERROR_SCRATCH_TOO_SMALL;
     if (tuning && !tuning_valid(tuning)) return ORN_ERROR_INVALID_VALUE;
+    const uint32_t n = params->width * params->height;
     const orn_tuning tn = tuning ? normalized(*tuning) : untuned(false);
     const int device = s->ctx->device;
     if (device < 0 || device >= kMaxDevices) return ORN_ERROR_INVALID_DEVICE;
@@ -2274,15 +2287,40 @@ orn_status orn_render_noalloc(orn_device_scene *s, const orn_constant_params *pa
     std::lock_guard<std::mutex> lock(g_scratch_mutex);
     ScratchSlot &sl = g_scratch[device];
     if (!sl.ptr) return ORN_ERROR_INVALID_DEVICE;  // set when the device was opened
-    uint32_t *queues = sl.ptr;
-    uint32_t *stage = sl.ptr + kScratchQueueWords;
-    if (++sl.epoch > 0xffffu) {  // tags wrap: clear every stage word an earlier call may have left
-        fill_u32_kernel<<<blocks_for(ORN_RENDER_SCRATCH_PIXELS, 256), 256, 0, st>>>(stage, ORN_RENDER_SCRATCH_PIXELS,
-                                                                                   0u);
-        sl.epoch = 1;
+    Scratch *const sc = sl.ptr;
+    auto next_epoch = [&]() {
+        if (++sl.epoch > 0xffffu) {  // tags wrap: clear every stage word an earlier call may have left
+            fill_u32_kernel<<<blocks_for(ORN_RENDER_SCRATCH_PIXELS, 256), 256, 0, st>>>(
+                sc->stage, ORN_RENDER_SCRATCH_PIXELS, 0u);
+            sl.epoch = 1;
+        }
+    };
+    float4 *const acc = reinterpret_cast<float4 *>(accumulation), *const fb = reinterpret_cast<float4 *>(framebuffer);
+    next_epoch();
+    // There is no earlier call to take costs from, so an order by cost comes
+    // from the call's own first eighth, as in a target's first render: 1,024
+    // instanced icospheres 1080p, 32 spp, 25.3 ms in tile order, 21.9 in jobs of
+    // two samples, 20.6 by cost; random spheres 64 spp 28.1 -> 25.7. Small
+    // images do not repay the second launch (see kCostOrderPixels), some
+    // larger ones neither (a Cornell box 512x512, 8 spp 1.18 -> 1.31), so only a
+    // tuning that asks for it gets it. Split pixels keep tile order: they end
+    // together without it.
+    const bool whole = tn.split_percent == 0u || tn.samples_per_job == 0u || tn.samples_per_job >= iterations;
+    const uint32_t tiles = blocks_for(params->width, kTile) * blocks_for(params->height, kTile);
+    if (tn.cost_order != 0u && whole && iterations >= kCostOrderSpp && n >= kCostOrderPixels &&
+        tiles <= kScratchTiles && splits_exactly(params->current_iteration, iterations)) {
+        const uint32_t first = iterations / 8u;
+        ORN_TRY(enqueue_render(s, params, first, tn, acc, rng, nullptr, sc->stage, sc->queues, sl.epoch, st, nullptr,
+                               sc->cost));
+        next_epoch();
+        enqueue_queue_order(params->width, params->height, sc->cost, sc->counts, sc->totals, sc->order, st);
+        orn_constant_params rest = *params;
+        rest.current_iteration = params->current_iteration + static_cast<float>(first);
+        ORN_TRY(enqueue_render(s, &rest, iterations - first, tn, acc, rng, fb, sc->stage, sc->queues, sl.epoch, st,
+                               sc->order, nullptr, sc->totals));
+        return ORN_OK;
     }
-    ORN_TRY(enqueue_render(s, params, iterations, tn, reinterpret_cast<float4 *>(accumulation), rng,
-                           reinterpret_cast<float4 *>(framebuffer), stage, queues, sl.epoch, st));
+    ORN_TRY(enqueue_render(s, params, iterations, tn, acc, rng, fb, sc->stage, sc->queues, sl.epoch, st));
     return ORN_OK;
 }
 
