@@ -1285,7 +1285,6 @@ orn_status validate(const orn_scene_desc *d, uint32_t *stack_slots)
     return ORN_OK;
 }
 
-
 orn_tuning default_tuning()
 {
     orn_tuning t{};

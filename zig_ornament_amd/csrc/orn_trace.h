@@ -67,7 +67,6 @@ struct DevScene {
     // reference's order.
     const char *__restrict__ search;
     uint32_t search_root;  // as the search tree's references go
-    uint32_t pad;
     float cull_rel, cull_abs;  // slack of the ordered search's distance cull (trav_cull)
     uint32_t plain_spheres;    // every sphere is scaled along the axes and moved (see sphere_leaf)
 };
@@ -353,7 +352,7 @@ __device__ __forceinline__ void pin_node(float4 &a, float4 &b, float4 &c, float4
 // Takes the next pending node off the lane's stack; false when none is left.
 // A BLAS is done when the stack is down to where it was on entering it (the
 // reference pushes a marker instead, bvh.wgsl:88-95).
-template <uint32_t F, uint32_t W>
+template <uint32_t F>
 __device__ __forceinline__ bool trav_pop(uint32_t *stack, uint32_t stride, Traversal &tr)
 {
     if (tr.top == 0u) return false;
@@ -443,7 +442,7 @@ __device__ __forceinline__ bool trav_internal(const DevScene &sc, float t_min, c
         const bool blas = (F & kHasMeshes) && tr.blas_top != kInTlas;
         const float4 *nd = (blas ? sc.blas4 : sc.tlas4) + 8u * tr.addr;
         if (bvh4_node(nd, stack, stride, cap, t_min, tr)) return true;
-        return trav_pop<F, W>(stack, stride, tr);
+        return trav_pop<F>(stack, stride, tr);
     }
     bool l, r;
     uint32_t left, right;
@@ -484,7 +483,7 @@ __device__ __forceinline__ bool trav_internal(const DevScene &sc, float t_min, c
         tr.addr = left_first ? left : right;
         return true;
     }
-    return trav_pop<F, W>(stack, stride, tr);
+    return trav_pop<F>(stack, stride, tr);
 }
 
 template <uint32_t F, uint32_t W>
@@ -563,7 +562,7 @@ __device__ __forceinline__ bool trav_leaf(const DevScene &sc, float t_min, const
             trav_behind(tr, t);
         }
     }
-    return trav_pop<F, W>(stack, stride, tr);
+    return trav_pop<F>(stack, stride, tr);
 }
 
 // The ray of a finished ordered search once more, in the reference's order
