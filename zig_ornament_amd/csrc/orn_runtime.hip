@@ -2795,7 +2795,8 @@ orn_status capture_batch(orn_batch *b)
         kp.order = b->order;
         kp.cost = b->cost;
     }
-    LaunchArgs a{kp, b->d_items, b->d_work, b->acc, b->rng, b->stage, b->queues, b->total_tiles, false, by_cost ? b->totals : nullptr};
+    LaunchArgs a{kp, b->d_items, b->d_work, b->acc, b->rng, b->stage, b->queues, b->total_tiles, false,
+                 by_cost ? b->totals : nullptr};
     ORN_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed));
     hipError_t e = hipMemcpyAsync(b->d_items, b->h_items, b->n * sizeof(BatchItem), hipMemcpyHostToDevice, st);
     if (e == hipSuccess && by_cost) {
