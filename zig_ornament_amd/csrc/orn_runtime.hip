@@ -1653,6 +1653,7 @@ public:
     std::vector<uint32_t> nodes;  // TLAS trees, then BLAS trees, in the given format
     std::vector<uint32_t> roots;  // search root reference of each TLAS root
     uint32_t slots = 1;           // traversal stack entries it needs, in any order of the children
+    SphereCull cull{};            // of a scene without meshes
 
     // `format`: bvh2_format() of the scene's launches, 2 or 3.
     explicit SearchTree(uint32_t format) : format_(format) {}
@@ -1663,6 +1664,7 @@ public:
         std::vector<orn_bvh_node> t = tlas;
         std::vector<uint32_t> b;  // the BLAS trees, from place 0 until they join the TLAS's
         std::vector<uint32_t> blas_root(d->blas_nodes_len, kEmptyRef), blas_slots(d->blas_nodes_len, 0u);
+        std::vector<MeshCore> core(d->blas_nodes_len);
         std::vector<orn_sah::Leaf> leaves, blas_leaves;
         std::vector<uint32_t> below(t.size(), 0u);  // stack entries a TLAS leaf's BLAS needs
         size_t collected = 0;
@@ -1672,6 +1674,8 @@ public:
             for (orn_sah::Leaf &l : leaves) {
                 const uint32_t idx = l.ref & ~kLeafRef;
                 orn_bvh_node nd = t[idx];
+                if (nd.node_type == 1u && format_ == 2u && !sphere_cull(d->transforms + 32 * size_t(nd.transform_id)))
+                    return false;
                 std::memcpy(nd.lmin_or_v0, l.box.lo, 12);  // the leaf's own box, in words not otherwise read
                 std::memcpy(nd.lmax_or_v1, l.box.hi, 12);
                 if (nd.node_type != 2u) {
@@ -1684,10 +1688,15 @@ public:
                     collect(d->blas_nodes, r, blas_leaves);
                     collected += blas_leaves.size();
                     if (collected > 2 * d->blas_nodes_len) return false;  // roots inside one another's trees
+                    core[r] = mesh_core(d->blas_nodes, blas_leaves);
                     if (!grow(blas_leaves, b, &blas_root[r])) return false;
                     blas_slots[r] = pending(b, blas_root[r], nullptr);
                 }
                 nd.left_or_custom_id = blas_root[r];
+                std::memcpy(nd.rmin_or_v2, core[r].centre, 12);  // more words not otherwise read
+                nd.rmax_or_v3[0] = core[r].radius2;
+                nd.rmax_or_v3[1] = kEtaNear * core[r].eta;
+                nd.rmax_or_v3[2] = kEtaFar * core[r].eta * core[r].size;
                 l.ref = kLeafRef | static_cast<uint32_t>(t.size());
                 t.push_back(nd);
                 below.push_back(1u + blas_slots[r]);
@@ -1756,8 +1765,197 @@ private:
         return true;
     }
 
+    // What a sphere adds to `cull` (cull_spheres): `inv` is the transform to
+    // its object space, x -> A x + b. False if the transform has no inverse.
+    bool sphere_cull(const float *inv)
+    {
+        double a[3][3], w[3][3], norm2 = 0.0, back2 = 0.0;  // A and its inverse, and their squared norms
+        for (int r = 0; r < 3; r++)
+            for (int c = 0; c < 3; c++) {
+                a[r][c] = inv[4 * c + r];
+                norm2 += a[r][c] * a[r][c];
+            }
+        double det = 0.0;
+        for (int c = 0; c < 3; c++) {
+            const int c1 = (c + 1) % 3, c2 = (c + 2) % 3;
+            for (int r = 0; r < 3; r++) {
+                const int r1 = (r + 1) % 3, r2 = (r + 2) % 3;
+                w[c][r] = a[r1][c1] * a[r2][c2] - a[r1][c2] * a[r2][c1];  // cofactor of a[r][c], transposed
+            }
+            det += a[0][c] * w[c][0];
+        }
+        double reach[3] = {}, origin = 0.0, fixed = 0.0, extent = 0.0;
+        for (int r = 0; r < 3; r++) {
+            double ext2 = 0.0, moved = 0.0, rows = 0.0;
+            for (int c = 0; c < 3; c++) {
+                w[r][c] /= det;
+                ext2 += w[r][c] * w[r][c];
+                moved += std::fabs(w[r][c] * inv[12 + c]);
+                rows += std::fabs(w[r][c]) * (std::fabs(a[c][0]) + std::fabs(a[c][1]) + std::fabs(a[c][2]));
+            }
+            reach[r] = std::sqrt(ext2);
+            back2 += ext2;
+            origin = std::max(origin, rows);
+            fixed = std::max(fixed, moved);
+            extent = std::max(extent, reach[r]);
+        }
+        if (!std::isfinite(origin + fixed + back2 + norm2)) return false;
+        bool axes = true;
+        double scale = 0.0;  // of a direction to object space
+        for (int r = 0; r < 3; r++)
+            for (int c = 0; c < 3; c++) {
+                if (r == c) scale = std::max(scale, std::fabs(a[r][c]));
+                else axes = axes && a[r][c] == 0.0;
+            }
+        if (!axes) scale = std::sqrt(norm2);
+        // X / 2 = 14 u (q^2 + 1) of the extent, q^2 + 1 <= (y scale)^2 + 2.03 y scale + 2.03 for y = |t d|;
+        // 4 u (|A| |o| + |b| + |t| |A| |d|) back in world space for the transform. 1.02 for the sums on the device.
+        const double u = kUnit, share = 14.0 * u * extent;
+        auto raise = [](float &f, double v) { f = std::max(f, static_cast<float>(1.02 * v)); };
+        raise(cull.fixed, 2.03 * share + 4.0 * u * fixed);
+        raise(cull.origin, 4.0 * u * origin);
+        raise(cull.dist, 2.03 * share * scale + 4.0 * u * origin);
+        raise(cull.dist2, 1.005 * share * scale * scale);
+        raise(cull.least_dir2, 1e-28 * back2);
+        return true;
+    }
+
+    // The core of a mesh (blas_slack): the ball around `centre` that a ray
+    // reaches only if it meets every triangle of the mesh at a determinant of at
+    // least kappa |d| |e1| |e2|. For a triangle whose edges meet at an angle of
+    // sine s, at a plane distance h from the centre and its vertex w from the foot
+    // of that distance, a ray nearly in its plane stays at least
+    //     h sqrt(1 - x^2) - x w - 2.1 kappa e / s,  x = 2 kappa / s^2
+    // away, less the rounding of o - v (20.2 u / s of the origin's distance, which
+    // the radius and the test on the device leave room for). kappa trades the
+    // ball against eta = 10.3 u / kappa.
+    // Round and convex meshes have a ball in their middle nearly as large as fits
+    // there. Open ones that face one way (a wall, a terrain) have one far in front
+    // of them, which rays reach that meet the surface steeply enough. Others (parts
+    // of several kinds in one mesh) may have none: their rays search all of it.
+    struct MeshCore {
+        float centre[3] = {}, radius2 = -1.0f, eta = 0.0f, size = 0.0f;
+    };
+    static MeshCore mesh_core(const orn_bvh_node *n, const std::vector<orn_sah::Leaf> &triangles)
+    {
+        constexpr int kKappas[] = {6, 8, 10, 12};  // kappa 2^-6 to 2^-12
+        constexpr int kRays = 256;                 // that the cores are compared over
+        constexpr double kFar = 64.0;              // mesh sizes between an open mesh and its core's centre
+        auto dot3 = [](const double *x, const double *y) { return x[0] * y[0] + x[1] * y[1] + x[2] * y[2]; };
+        auto cross3 = [](const double *x, const double *y, double *z) {
+            for (int a = 0; a < 3; a++) z[a] = x[(a + 1) % 3] * y[(a + 2) % 3] - x[(a + 2) % 3] * y[(a + 1) % 3];
+        };
+        orn_sah::Box box = orn_sah::Box::empty();
+        double facing[3] = {}, area_sum = 0.0;
+        for (const orn_sah::Leaf &l : triangles) {
+            const orn_bvh_node &nd = n[l.ref & ~kLeafRef];
+            double e1[3], e2[3], c[3];
+            for (int a = 0; a < 3; a++) {
+                e1[a] = double(nd.lmax_or_v1[a]) - nd.lmin_or_v0[a];
+                e2[a] = double(nd.rmin_or_v2[a]) - nd.lmin_or_v0[a];
+            }
+            cross3(e1, e2, c);
+            for (int a = 0; a < 3; a++) facing[a] += c[a];
+            area_sum += std::sqrt(dot3(c, c));
+            for (const float *v : {nd.lmin_or_v0, nd.lmax_or_v1, nd.rmin_or_v2}) box.grow(box_of(v, v));
+        }
+        double half = 0.0;
+        float middle[3], front[3];
+        for (int a = 0; a < 3; a++) {
+            middle[a] = 0.5f * box.lo[a] + 0.5f * box.hi[a];
+            half = std::hypot(half, 0.5 * (double(box.hi[a]) - box.lo[a]));
+        }
+        const double faced = std::sqrt(dot3(facing, facing));
+        for (int a = 0; a < 3; a++) front[a] = static_cast<float>(middle[a] + kFar * half * facing[a] / faced);
+
+        MeshCore best;
+        int met = 0;  // rays that reach its ball
+        auto consider = [&](const float *centre) {
+            double radius[4], least_sine = 1.0, size = 0.0;
+            if (!core_radii(n, triangles, centre, kKappas, radius, &least_sine, &size)) return;
+            const double u = kUnit, tau = 20.2 * u / least_sine;
+            for (int k = 0; k < 4; k++) {
+                const double eta = 10.3 * u * std::ldexp(1.0, kKappas[k]), r = radius[k] - tau * size;
+                // the test on the device leaves eta / kEtaBall of the origin's distance for its rounding and tau
+                if (30.0 * u + 1.01 * tau > eta / kEtaBall || !(r >= kLeastLength && r <= kMostLength)) continue;
+                const double r2 = r * r * (1.0 - tau) * (1.0 - 16.0 * u);
+                uint32_t seed = 1u;  // rays through points of the mesh, in any direction
+                auto draw = [&seed] {
+                    seed = seed * 1664525u + 1013904223u;
+                    return double(seed >> 8) / 16777216.0;
+                };
+                int count = 0;
+                for (int i = 0; i < kRays; i++) {
+                    const orn_bvh_node &nd = n[triangles[size_t(draw() * double(triangles.size()))].ref & ~kLeafRef];
+                    const double z = 2.0 * draw() - 1.0, phi = 6.283185307179586 * draw(), ring = std::sqrt(1.0 - z * z);
+                    const double d[3] = {ring * std::cos(phi), ring * std::sin(phi), z};
+                    double p[3], off[3];
+                    for (int a = 0; a < 3; a++)
+                        p[a] = (double(nd.lmin_or_v0[a]) + nd.lmax_or_v1[a] + nd.rmin_or_v2[a]) / 3.0 - centre[a];
+                    cross3(p, d, off);
+                    count += dot3(off, off) + eta / kEtaBall * dot3(p, p) < r2;
+                }
+                // a smaller kappa widens every cull fourfold: for an eighth more rays only
+                if (count <= met + kRays / 8) continue;
+                met = count;
+                for (int a = 0; a < 3; a++) best.centre[a] = centre[a];
+                best.radius2 = static_cast<float>(r2);
+                best.eta = static_cast<float>(eta);
+                best.size = static_cast<float>(size * (1.0 + 4.0 * u));
+            }
+        };
+        consider(middle);
+        if (faced > 0.5 * area_sum) consider(front);
+        return best;
+    }
+
+    static constexpr double kLeastLength = 1e-12, kMostLength = 1e12;  // products neither under- nor overflow
+
+    // The ball's radius for each kappa 2^-k, the least sine of an angle at a first
+    // vertex and the farthest vertex. False if a mesh can have no core.
+    static bool core_radii(const orn_bvh_node *n, const std::vector<orn_sah::Leaf> &triangles, const float *centre,
+                           const int (&kappas)[4], double (&radius)[4], double *least_sine, double *size)
+    {
+        std::fill(radius, radius + 4, std::numeric_limits<double>::infinity());
+        for (const orn_sah::Leaf &l : triangles) {
+            const orn_bvh_node &nd = n[l.ref & ~kLeafRef];
+            double v[3][3], e1[3], e2[3], far2 = 0.0, l1 = 0.0, l2 = 0.0, area = 0.0, h = 0.0;
+            for (int a = 0; a < 3; a++) {
+                v[0][a] = double(nd.lmin_or_v0[a]) - centre[a];
+                v[1][a] = double(nd.lmax_or_v1[a]) - centre[a];
+                v[2][a] = double(nd.rmin_or_v2[a]) - centre[a];
+                e1[a] = v[1][a] - v[0][a];
+                e2[a] = v[2][a] - v[0][a];
+                l1 += e1[a] * e1[a];
+                l2 += e2[a] * e2[a];
+            }
+            for (const auto &p : v) far2 = std::max(far2, p[0] * p[0] + p[1] * p[1] + p[2] * p[2]);
+            *size = std::max(*size, std::sqrt(far2));
+            if (l1 == 0.0 || l2 == 0.0) continue;  // its determinant is 0 and its t NaN: never hit
+            l1 = std::sqrt(l1);
+            l2 = std::sqrt(l2);
+            for (int a = 0; a < 3; a++) {
+                const double c = e1[(a + 1) % 3] * e2[(a + 2) % 3] - e1[(a + 2) % 3] * e2[(a + 1) % 3];
+                area += c * c;
+                h += c * v[0][a];
+            }
+            area = std::sqrt(area);
+            const double sine = area / (l1 * l2);
+            if (!(std::min(l1, l2) >= kLeastLength) || !(sine > 0.0)) return false;
+            h = std::fabs(h) / area;
+            *least_sine = std::min(*least_sine, sine);
+            const double w = std::sqrt(std::max(0.0, v[0][0] * v[0][0] + v[0][1] * v[0][1] + v[0][2] * v[0][2] - h * h));
+            for (int k = 0; k < 4; k++) {
+                const double kappa = std::ldexp(1.0, -kappas[k]), x = 2.0 * kappa / (sine * sine);
+                const double r = x > 0.7 ? -1.0 : h * std::sqrt(1.0 - x * x) - x * w - 2.1 * kappa * std::max(l1, l2) / sine;
+                radius[k] = std::min(radius[k], r);
+            }
+        }
+        return *size <= kMostLength;
+    }
+
     // The leaves below `root` with the boxes their parents hold for them (a
-    // root that is a leaf has none that is tested: its own words stand in).
+    // root that is a leaf has none that is tested: all of space).
     static void collect(const orn_bvh_node *n, uint32_t root, std::vector<orn_sah::Leaf> &out)
     {
         std::vector<uint32_t> todo;
@@ -1765,7 +1963,8 @@ private:
             if (n[i].node_type == 0u) todo.push_back(i);
             else out.push_back({b, kLeafRef | i});
         };
-        visit(root, box_of(n[root].lmin_or_v0, n[root].lmax_or_v1));
+        constexpr float far = std::numeric_limits<float>::max();
+        visit(root, orn_sah::Box{{-far, -far, -far}, {far, far, far}});
         while (!todo.empty()) {
             const orn_bvh_node &nd = n[todo.back()];
             todo.pop_back();
@@ -1926,11 +2125,7 @@ orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots
         ds.search_root = search_root[0];
         if (!ordered) s->features |= kNoSearchTree;
         s->traversal_slots = ordered ? std::max(slots, search.slots) : slots;
-        float size = 0.0f;  // largest coordinate of the scene
-        for (int a = 0; a < 3; a++)
-            size = std::fmax(size, std::fmax(std::fabs(s->bounds_lo[a]), std::fabs(s->bounds_hi[a])));
-        ds.cull_rel = kCullRel;
-        ds.cull_abs = kCullUlp * size;
+        ds.cull = search.cull;
         // one array: the BLAS nodes behind the TLAS's
         const size_t tlas_n = t2.size();
         if (tlas_n + b2.size() >= kLeafRef) return fail(ORN_ERROR_OUT_OF_MEMORY);

@@ -17,9 +17,12 @@ namespace orn {
 constexpr uint32_t kFinishedTraverseBlas = 0xffffffffu;  // pathtracer.wgsl:19
 constexpr uint32_t kInTlas = 0xffffffffu;
 constexpr float kTMaxInit = 3.40282e+38f;                 // bvh.wgsl:23
-// slack of the ordered search's distance cull (trav_cull)
-constexpr float kCullRel = 1.0f / 512.0f;    // of t
-constexpr float kCullUlp = 1.0f / 2097152.0f;  // of coordinates: 4 ulp
+// The ordered search's distance culls (cull_spheres, blas_slack)
+constexpr float kUnit = 5.9604645e-8f;            // unit roundoff
+constexpr float kCullOffset = 4.0f * kUnit;       // of |o * inv|: the slab distances' rounding
+constexpr float kCullRel = 1.0f + 16.0f * kUnit;  // of t
+constexpr float kLeastDir2 = 3.2e-10f;  // |d|^2 from which safe_invdir leaves the largest component alone
+constexpr float kEtaNear = 4.5f, kEtaFar = 8.9f, kEtaBall = 8.0f;
 
 // One texture in the texel pool. format: components | (hdr << 8)
 struct DevTexture {
@@ -34,6 +37,13 @@ struct DevTexture {
 // into the BVH2 array of the same level) or an empty slot.
 constexpr uint32_t kLeafRef = 0x80000000u;
 constexpr uint32_t kEmptyRef = 0xfffffffeu;
+
+// How far in front of its box rounding can put a sphere's distance, over every
+// sphere of a scene without meshes (SearchTree::sphere_cull, cull_spheres).
+struct SphereCull {
+    float fixed, origin, dist, dist2;  // of 1, the ray's origin, and the distance and its square
+    float least_dir2;                  // |d|^2 below which squares underflow
+};
 
 // The bound buffers of pathtracer.wgsl:7-17, resident in HBM, plus the
 // derived BVH4 arrays (8 float4 = 128 B per node: children's min x, y, z,
@@ -67,8 +77,8 @@ struct DevScene {
     // reference's order.
     const char *__restrict__ search;
     uint32_t search_root;  // as the search tree's references go
-    float cull_rel, cull_abs;  // slack of the ordered search's distance cull (trav_cull)
-    uint32_t plain_spheres;    // every sphere is scaled along the axes and moved (see sphere_leaf)
+    uint32_t plain_spheres;  // every sphere is scaled along the axes and moved (see sphere_leaf)
+    SphereCull cull;
 };
 
 // An internal node of the search tree of a scene without meshes: per axis the
@@ -278,21 +288,34 @@ constexpr bool is_search_format(uint32_t w) { return w == 2u || w == 3u; }
 //    above then pass too, in either tree, and no other primitive is visited
 //    by either search.
 //  * The reference returns the smallest t over the primitives in reach, the
-//    first visited among equal ones, unless rounding put that t in front of
-//    the primitive's own leaf box (`early`: half of all hits on a flat,
+//    first visited among equal ones, unless that t lies in front of the
+//    primitive's own boxes (rounding: half of all hits on a flat,
 //    axis-aligned wall) and another hit lies between the two: the other one,
-//    met first, culls the box. The ordered search sees both cases, a tie
-//    with the best t and another hit just behind an early one: they set
-//    `redo`, and the ray is searched again in the reference's order
-//    (trav_redo; about 2 in 1e5 rays on instanced icospheres).
-//  * So that a primitive whose t was rounded in front of its box is still
-//    visited, and so is a hit behind it, boxes and primitives are culled
-//    only beyond t_cull, a little past the best t and its box.
+//    met first, culls the boxes. The ordered search sees both cases, a tie
+//    with the best t and another hit in front of the best one's boxes: they
+//    set `redo`, and the ray is searched again in the reference's order
+//    (trav_redo).
+//  * That holds as long as every primitive in reach is visited whose t is no
+//    larger than the best one's, or than where the best one's boxes begin
+//    (`near_best`). So a box is culled only beyond t_cull, which lies past
+//    both by as much as rounding can put a primitive's t in front of its
+//    box. For spheres that is bounded by the scene (cull_spheres).
+//    For triangles it is bounded only where the ray is not nearly in the
+//    triangle's plane: there the determinant, which the reference does not
+//    test, is rounding noise, and so is t. A BLAS is culled where its mesh's
+//    core rules such triangles out (blas_slack), and searched whole where not;
+//    between BLASes, whose meshes a ray has not yet been compared with,
+//    nothing is culled.
 // The search is bound by the vector instructions of its node visits, so fewer
-// visits are time: random spheres 1920x1080, 64 spp, 52 -> 33 ms; 1,024
-// instanced icospheres, 32 spp, 40 -> 30 ms; a batch of 16 instanced scenes
-// 25 -> 15 ms (with the same launch shapes, readback included). Scenes whose
-// arrays do not have nested boxes (SearchTree::build) have no search tree.
+// visits are time: random spheres 1920x1080, 64 spp, 52 -> 33 ms with it. The
+// kernels of mesh scenes in the reference's order and in this one: 1,024 instanced
+// icospheres 1080p, 32 spp, 33.5 -> 22.7 ms, textured, metal and glass icospheres
+// 700x700, 8 spp, 6.5 -> 3.76, 16 images of such scenes 9.7 -> 6.95, the Cornell
+// box 256x256, 16 spp, 1.58 -> 1.46, 200 tori (no core) 960x540, 8 spp, 32.2 -> 29.1.
+// (A cull by distance at every box would take the icospheres 18.5 ms and miss hits;
+// the instances behind the hit cost 2.1, the slack's arithmetic 0.9 and rays that
+// pass by the core 1.4.) Scenes whose arrays do not have nested boxes (SearchTree::build) have no search
+// tree.
 struct Traversal {
     Ray ray;        // the ray in object space, inside a BLAS
     f3 inv, ox;     // safe_invdir(d) and -o * inv of the ray in the current space
@@ -300,13 +323,14 @@ struct Traversal {
     uint32_t sx, sy, sz;  // W = 2: plane offsets of a SearchNode by the signs of inv
     float t_max;
     float t_cull;     // search tree: boxes and hits beyond it are skipped
+    float near_best;  // search tree: where the boxes of the closest hit begin
     float mesh_near;  // search tree: where the ray enters the box of the instance it is in
+    float slack;      // search tree: how far past the best hit the BLAS it is in is searched
     uint32_t addr;  // next node to visit
     uint32_t top;   // pending entries in the LDS column
     uint32_t material_index, inv_tid;  // of the mesh being traversed
     uint32_t blas_top;  // `top` when the ray entered the BLAS it is in (kInTlas: none)
     bool hit;
-    bool early;  // search tree: the closest hit lies in front of its own box
     bool redo;   // search tree: the closest hit needs the reference's order (see above)
     Hit h;
 };
@@ -330,8 +354,9 @@ __device__ __forceinline__ void trav_begin(uint32_t root, const Ray &world, Trav
     tr.wox = tr.ox;
     tr.t_max = kTMaxInit;
     tr.t_cull = kTMaxInit;
+    tr.near_best = 0.0f;
     tr.mesh_near = 0.0f;
-    tr.early = false;
+    tr.slack = 0.0f;
     tr.redo = false;
     tr.addr = root;
     tr.top = 0u;
@@ -360,6 +385,7 @@ __device__ __forceinline__ bool trav_pop(uint32_t *stack, uint32_t stride, Trave
         // back in the TLAS: the world-space ray's reciprocal, kept from
         // trav_begin
         tr.blas_top = kInTlas;
+        tr.t_cull = kTMaxInit;
         tr.inv = tr.winv;
         tr.ox = tr.wox;
     }
@@ -402,30 +428,81 @@ __device__ __forceinline__ bool bvh4_node(const float4 *nd, uint32_t *stack, uin
     return true;
 }
 
-// A new closest hit at t after one at t_old, its boxes entered at near_t: the
-// distance beyond which boxes are culled from now on, and whether rounding
-// put t in front of its boxes. The slack covers the rounding of t and of the
-// slab distances: a share of t (a near-tangent sphere hit is off by up to
-// sqrt(8 ulp) of the distance) and an absolute part for the cancellation in
-// o - box of coordinates up to the scene's (or the origin's) size, over the
-// direction.
-template <uint32_t F>
-__device__ __forceinline__ void trav_cull(const DevScene &sc, Traversal &tr, float t, float t_old, float near_t)
+__device__ __forceinline__ float max_abs(f3 a) { return fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fabsf(a.z)); }
+
+// sqrt to within an ulp, for bounds that have room for it
+ORN_HD float sqrt_near(float x)
 {
-    const f3 wi = (F & kHasMeshes) ? tr.winv : tr.inv;
-    const float inv = fmaxf(fmaxf(fabsf(wi.x), fabsf(wi.y)), fabsf(wi.z));
-    float off = fmaxf(fmaxf(fabsf(tr.ox.x), fabsf(tr.ox.y)), fabsf(tr.ox.z));
-    if (F & kHasMeshes) off = fmaxf(off, fmaxf(fmaxf(fabsf(tr.wox.x), fabsf(tr.wox.y)), fabsf(tr.wox.z)));
-    const float slack = fmaf(sc.cull_rel, fabsf(t), fmaf(sc.cull_abs, inv, kCullUlp * off));
-    tr.t_cull = fmaxf(t, near_t) + slack;
-    tr.early = near_t > t;
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __builtin_amdgcn_sqrtf(x);
+#else
+    return sqrtf(x);
+#endif
+}
+
+// What t_cull is measured from: the best hit, where its boxes begin, and the
+// size of any distance in front of those.
+__device__ __forceinline__ float cull_from(const Traversal &tr, float t_min)
+{
+    return fmaxf(fmaxf(tr.t_max, tr.near_best), fabsf(t_min));
+}
+
+// t_cull in a scene of spheres alone. With o, d the ray in a sphere's object
+// space and q = |o|, the terms of sphere_hit's discriminant are off by at most
+// u (17 q^2 + 6) |d|^2 (u: unit roundoff), and the root taken from them puts
+// the point o + t d outside of the unit sphere by at most X / 2 with
+// X = 28 u (q^2 + 1), near-tangent hits included: there t is off along the
+// surface, not away from it. q itself is at most 1.002 (|t d| + 1.01). In
+// world space that and the rounding of the transform bound how far the point
+// lies outside of the sphere's box (SphereCull, by SearchTree::sphere_cull),
+// and the slab distance of the box is in front of t by no more than that over
+// the direction's smallest component. The bound grows with t, so it is taken
+// for the largest t that matters.
+__device__ __forceinline__ void cull_spheres(const DevScene &sc, const Ray &world, float t_min, Traversal &tr)
+{
+    const float from = cull_from(tr, t_min), dd = dot(world.d, world.d), y = from * sqrt_near(dd);
+    const float out = fmaf(y, fmaf(y, sc.cull.dist2, sc.cull.dist), fmaf(max_abs(world.o), sc.cull.origin, sc.cull.fixed));
+    const float slack = fmaf(max_abs(tr.inv), out, kCullOffset * max_abs(tr.ox));
+    // (fminf drops a NaN, and infinite coordinates cull nothing)
+    tr.t_cull = dd >= sc.cull.least_dir2 ? fminf(fmaf(from, kCullRel, slack), kTMaxInit) : kTMaxInit;
+}
+
+// The slack of a BLAS for the object-space ray in `tr`; infinite where the ray
+// may lie nearly in the plane of one of the mesh's triangles. n2 and n3 are
+// the mesh leaf's words: the core's centre c, its squared radius r2, and eta
+// (times kEtaNear, and times kEtaFar and the mesh's size; SearchTree::mesh_core).
+// A triangle hit (u, v and t accepted) whose determinant is below kappa |d|
+// |e1| |e2| lies nearly in the ray's plane, so the ray passes c at a distance
+// of at least the triangle plane's, less what the core leaves for it. A ray
+// that comes closer to c meets every triangle at a larger determinant, where
+// rounding moves u, v and t by at most eta (1 + |o - v| / |e|), so that the
+// slab distance of the triangle's box is in front of t by no more than eta
+// (4.5 |o - c| + 8.9 R) over the direction's smallest component, in front of
+// which slab distances round by a few units of o * inv.
+__device__ __forceinline__ float blas_slack(float4 n2, float4 n3, const Traversal &tr)
+{
+    const f3 p = tr.ray.o - xyz(n2);
+    const float a = dot(p, p), b = dot(p, tr.ray.d), c = dot(tr.ray.d, tr.ray.d), ac = a * c;
+    const bool inside = fmaf(ac, n3.y * (1.0f / (kEtaNear * kEtaBall)), ac - b * b) < n3.x * c;
+    const float slack = fmaf(max_abs(tr.inv), fmaf(n3.y, sqrt_near(a), n3.z), kCullOffset * max_abs(tr.ox));
+    return inside && c >= kLeastDir2 ? slack : __builtin_inff();
+}
+__device__ __forceinline__ float blas_cull(const Traversal &tr, float t_min)
+{
+    return fminf(fmaf(cull_from(tr, t_min), kCullRel, tr.slack), kTMaxInit);
+}
+
+// A new closest hit (tr.t_max) after one at t_old, its boxes entered at near_t.
+__device__ __forceinline__ void trav_nearer(Traversal &tr, float t_old, float near_t)
+{
+    tr.near_best = near_t;
     tr.redo = near_t > t_old;
 }
 
-// A hit at t no closer than the best one, but not beyond t_cull.
+// A hit at t no closer than the best one.
 __device__ __forceinline__ void trav_behind(Traversal &tr, float t)
 {
-    if (tr.early || t == tr.t_max) tr.redo = true;
+    if (t < tr.near_best || t == tr.t_max) tr.redo = true;
 }
 
 // Node references carry kLeafRef when they name a leaf (in the BVH4 by
@@ -517,7 +594,8 @@ __device__ __forceinline__ bool trav_leaf(const DevScene &sc, float t_min, const
                 float near_t;  // the leaf's own box is kept in the unused words of the leaf
                 (void)aabb_hit(make_float3(n0.x, n0.y, n0.z), make_float3(n1.x, n1.y, n1.z), tr.inv, tr.ox, t_min,
                                tr.t_max, near_t);
-                trav_cull<F>(sc, tr, t, t_old, near_t);
+                trav_nearer(tr, t_old, near_t);
+                if constexpr (W == 2u) cull_spheres(sc, world, t_min, tr);
             }
         } else if (ORD && ok) {
             trav_behind(tr, t);
@@ -532,6 +610,10 @@ __device__ __forceinline__ bool trav_leaf(const DevScene &sc, float t_min, const
         tr.ray = xform_ray(sc.transforms + 4u * tr.inv_tid, world);
         tr.inv = safe_invdir(tr.ray.d);
         tr.ox = (-tr.ray.o) * tr.inv;
+        if constexpr (ORD) {
+            tr.slack = blas_slack(n2, n3, tr);
+            tr.t_cull = blas_cull(tr, t_min);
+        }
         tr.addr = as_u32(n0.w);
         return true;
     } else if ((F & kHasMeshes) && type == 3u) {
@@ -556,7 +638,8 @@ __device__ __forceinline__ bool trav_leaf(const DevScene &sc, float t_min, const
                                make_float3(fmaxf(fmaxf(n0.x, n1.x), n2.x), fmaxf(fmaxf(n0.y, n1.y), n2.y),
                                            fmaxf(fmaxf(n0.z, n1.z), n2.z)),
                                tr.inv, tr.ox, t_min, tr.t_max, near_t);
-                trav_cull<F>(sc, tr, t, t_old, fmaxf(near_t, tr.mesh_near));
+                trav_nearer(tr, t_old, fmaxf(near_t, tr.mesh_near));
+                tr.t_cull = blas_cull(tr, t_min);
             }
         } else if (ORD && ok) {
             trav_behind(tr, t);
