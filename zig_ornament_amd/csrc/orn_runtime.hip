@@ -1648,6 +1648,9 @@ void fill_sphere_leaves(const orn_scene_desc *d, std::vector<orn_bvh_node> &node
 // them: finite, each containing the boxes below it, a triangle's own spanning
 // its vertices, every node under one parent. Arrays that are not so keep the
 // reference's order throughout (build returns false and leaves them alone).
+// A sphere's box need not hold the sphere, nor an instance's box its mesh
+// (transforms moved under kept boxes): what a sphere's box leaves out widens
+// the cull (sphere_cull), and instances' boxes cull nothing.
 class SearchTree {
 public:
     std::vector<uint32_t> nodes;  // TLAS trees, then BLAS trees, in the given format
@@ -1674,7 +1677,7 @@ public:
             for (orn_sah::Leaf &l : leaves) {
                 const uint32_t idx = l.ref & ~kLeafRef;
                 orn_bvh_node nd = t[idx];
-                if (nd.node_type == 1u && format_ == 2u && !sphere_cull(d->transforms + 32 * size_t(nd.transform_id)))
+                if (nd.node_type == 1u && format_ == 2u && !sphere_cull(d->transforms + 32 * size_t(nd.transform_id), l.box))
                     return false;
                 std::memcpy(nd.lmin_or_v0, l.box.lo, 12);  // the leaf's own box, in words not otherwise read
                 std::memcpy(nd.lmax_or_v1, l.box.hi, 12);
@@ -1766,8 +1769,9 @@ private:
     }
 
     // What a sphere adds to `cull` (cull_spheres): `inv` is the transform to
-    // its object space, x -> A x + b. False if the transform has no inverse.
-    bool sphere_cull(const float *inv)
+    // its object space, x -> A x + b, `box` the box that rays test for it, which
+    // may leave out some of it. False if the transform has no inverse.
+    bool sphere_cull(const float *inv, const orn_sah::Box &box)
     {
         double a[3][3], w[3][3], norm2 = 0.0, back2 = 0.0;  // A and its inverse, and their squared norms
         for (int r = 0; r < 3; r++)
@@ -1784,11 +1788,12 @@ private:
             }
             det += a[0][c] * w[c][0];
         }
-        double reach[3] = {}, origin = 0.0, fixed = 0.0, extent = 0.0;
+        double reach[3] = {}, origin = 0.0, fixed = 0.0, extent = 0.0, miss = 0.0;
         for (int r = 0; r < 3; r++) {
-            double ext2 = 0.0, moved = 0.0, rows = 0.0;
+            double centre = 0.0, ext2 = 0.0, moved = 0.0, rows = 0.0;
             for (int c = 0; c < 3; c++) {
                 w[r][c] /= det;
+                centre -= w[r][c] * inv[12 + c];
                 ext2 += w[r][c] * w[r][c];
                 moved += std::fabs(w[r][c] * inv[12 + c]);
                 rows += std::fabs(w[r][c]) * (std::fabs(a[c][0]) + std::fabs(a[c][1]) + std::fabs(a[c][2]));
@@ -1798,8 +1803,9 @@ private:
             origin = std::max(origin, rows);
             fixed = std::max(fixed, moved);
             extent = std::max(extent, reach[r]);
+            miss = std::max({miss, box.lo[r] - (centre - reach[r]), centre + reach[r] - box.hi[r]});
         }
-        if (!std::isfinite(origin + fixed + back2 + norm2)) return false;
+        if (!std::isfinite(origin + fixed + back2 + norm2 + miss)) return false;
         bool axes = true;
         double scale = 0.0;  // of a direction to object space
         for (int r = 0; r < 3; r++)
@@ -1812,7 +1818,7 @@ private:
         // 4 u (|A| |o| + |b| + |t| |A| |d|) back in world space for the transform. 1.02 for the sums on the device.
         const double u = kUnit, share = 14.0 * u * extent;
         auto raise = [](float &f, double v) { f = std::max(f, static_cast<float>(1.02 * v)); };
-        raise(cull.fixed, 2.03 * share + 4.0 * u * fixed);
+        raise(cull.fixed, 2.03 * share + 4.0 * u * fixed + miss);
         raise(cull.origin, 4.0 * u * origin);
         raise(cull.dist, 2.03 * share * scale + 4.0 * u * origin);
         raise(cull.dist2, 1.005 * share * scale * scale);

@@ -453,11 +453,12 @@ __device__ __forceinline__ float cull_from(const Traversal &tr, float t_min)
 // the point o + t d outside of the unit sphere by at most X / 2 with
 // X = 28 u (q^2 + 1), near-tangent hits included: there t is off along the
 // surface, not away from it. q itself is at most 1.002 (|t d| + 1.01). In
-// world space that and the rounding of the transform bound how far the point
-// lies outside of the sphere's box (SphereCull, by SearchTree::sphere_cull),
-// and the slab distance of the box is in front of t by no more than that over
-// the direction's smallest component. The bound grows with t, so it is taken
-// for the largest t that matters.
+// world space that, the rounding of the transform and what the sphere's box
+// leaves out of the sphere bound how far the point lies outside of the box
+// (SphereCull, by SearchTree::sphere_cull), and the slab distance of the box
+// is in front of t by no more than that over the direction's smallest
+// component. The bound grows with t, so it is taken for the largest t that
+// matters.
 __device__ __forceinline__ void cull_spheres(const DevScene &sc, const Ray &world, float t_min, Traversal &tr)
 {
     const float from = cull_from(tr, t_min), dd = dot(world.d, world.d), y = from * sqrt_near(dd);
