@@ -1404,29 +1404,32 @@ template <uint32_t F, uint32_t W, bool BATCH, bool POOL>
 hipError_t launch_render_k(uint32_t per_cu, uint32_t cus, size_t lds, hipStream_t st, const DevScene &ds,
                            const LaunchArgs &a)
 {
-    if (per_cu == 0) {
-        int blocks = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, render_kernel<F, W, BATCH, POOL>, kBlock, lds) !=
-                hipSuccess ||
-            blocks < 1) {
-            (void)hipGetLastError();  // the launch below reports its own errors
-            blocks = 1;
-        }
-        per_cu = static_cast<uint32_t>(blocks);
+    int blocks = 0;  // that can be resident on a CU
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, render_kernel<F, W, BATCH, POOL>, kBlock, lds) !=
+            hipSuccess ||
+        blocks < 1) {
+        (void)hipGetLastError();  // the launch below reports its own errors
+        blocks = 1;
     }
-    uint32_t grid = std::max(kXcds, cus * per_cu / kXcds * kXcds);
+    auto groups = [cus](uint32_t n) { return std::max(kXcds, cus * n / kXcds * kXcds); };
+    uint32_t resident = groups(static_cast<uint32_t>(blocks));
+    uint32_t grid = per_cu == 0 ? resident : groups(per_cu);
+    resident = std::min(resident, grid);
     // A pixel is one lane's work from its first sample to its last, so an image
     // of fewer pixels than lanes leaves the choice between few full waves and
     // many sparse ones. In sparse waves a lane waits for fewer others at leaf
     // and shading rounds, but those rounds are issued once per wave, so the
-    // SIMDs must have the issue slots: up to 8 lanes of every resident wave.
+    // SIMDs must have the issue slots: up to 8 lanes of every resident wave. (A
+    // tuning may launch more workgroups than fit: those run when the pixels are
+    // gone, and counting their lanes left the others sparse: random spheres 500x500,
+    // 8 spp, in 32 workgroups per CU 2.68 ms, now 1.07.)
     // 8 spp, full -> sparse: instanced icospheres 64x64 1.64 -> 0.92 ms,
     // 160x160 1.91 -> 1.36; random spheres 128x128 0.97 -> 0.75, 160x160 0.94 ->
     // 0.85; Cornell box (every path bounces to its full depth) 96x96 0.86 ->
     // 0.65, 181x181 0.85 -> 0.87. Above that the box loses more than the others
     // gain (200x200 at 12 lanes: 0.83 -> 0.96, icospheres 1.83 -> 1.50).
     KernelParams kp = a.kp;
-    const uint32_t per_wave = blocks_for(kp.pixels, grid * (kBlock / 64u));
+    const uint32_t per_wave = blocks_for(kp.pixels, resident * (kBlock / 64u));
     kp.lanes = POOL || per_wave > kSparseLanes ? 64u : blocks_for(per_wave, kLaneStep) * kLaneStep;
     if (kp.lanes == 64u) {
         grid = std::min(grid, blocks_for(a.total_tiles, kXcds) * kXcds);
@@ -1436,7 +1439,8 @@ hipError_t launch_render_k(uint32_t per_cu, uint32_t cus, size_t lds, hipStream_
     }
     const bool whole = kp.split_pct == 0u || (!BATCH && kp.chunks == 1u);
     kp.heavy = !POOL && kp.lanes == 64u && whole && a.totals ? 1u : 0u;
-    start_queues_kernel<<<1, 64 * kXcds, 0, st>>>(a.queues, kp.heavy ? a.totals : nullptr, grid * kBlock);
+    start_queues_kernel<<<1, 64 * kXcds, 0, st>>>(a.queues, kp.heavy ? a.totals : nullptr,
+                                                 std::min(grid, resident) * kBlock);
     render_kernel<F, W, BATCH, POOL>
         <<<grid, kBlock, lds, st>>>(ds, kp, a.items, a.work, a.acc, a.rng, a.stage, a.queues);
     return hipGetLastError();
