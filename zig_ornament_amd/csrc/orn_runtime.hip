@@ -2372,9 +2372,8 @@ hipError_t enqueue_render(orn_device_scene *s, const orn_constant_params *params
     return hipGetLastError();
 }
 
-// Buffers of a target's cost-ordered queues, allocated on first use; the
-// costs start at zero.
-hipError_t ensure_cost_order(orn_target *t, hipStream_t st)
+// Buffers of a target's cost-ordered queues, allocated on first use.
+hipError_t ensure_cost_order(orn_target *t)
 {
     if (t->cost) return hipSuccess;
     const uint32_t n = t->width * t->height;
@@ -2392,9 +2391,8 @@ hipError_t ensure_cost_order(orn_target *t, hipStream_t st)
         t->cost = t->order = t->counts = t->totals = nullptr;
         return e;
     }
-    fill_u32_kernel<<<blocks_for(n, 256), 256, 0, st>>>(t->cost, n, 0u);
     t->costs_recorded = false;
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 // The queue order of an image's next render from the costs its previous
@@ -2433,7 +2431,7 @@ orn_status orn_render_async(orn_target *t, const orn_constant_params *params, ui
     next_epoch();
     orn_tuning tuning = t->tuned ? t->tuning : untuned(iterations >= kCostOrderSpp && n >= kCostOrderPixels);
     if (tuning.cost_order != 0u) {
-        const hipError_t e = ensure_cost_order(t, st);
+        const hipError_t e = ensure_cost_order(t);
         if (e != hipSuccess && t->tuned) return from_hip(e);
         if (e != hipSuccess) {  // the order was not asked for
             tuning.cost_order = 0u;
@@ -2441,6 +2439,9 @@ orn_status orn_render_async(orn_target *t, const orn_constant_params *params, ui
         }
     }
     const bool by_cost = tuning.cost_order != 0u;
+    // jobs add to the costs, so a first recording starts from none (the buffer
+    // may be new, or hold those of renders before a tuning was set)
+    if (by_cost && !t->costs_recorded) fill_u32_kernel<<<blocks_for(n, 256), 256, 0, st>>>(t->cost, n, 0u);
     ORN_TRY(hipEventRecord(t->ev_start, st));
     const uint32_t *order = nullptr;
     if (by_cost && t->costs_recorded) {
