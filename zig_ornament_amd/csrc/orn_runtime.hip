@@ -3379,10 +3379,11 @@ std::string scene_class(const orn_device_scene *s, uint64_t pixels, uint32_t spp
                         uint32_t flags)
 {
     char key[256];
-    std::snprintf(key, sizeof(key), "%s|features%u|tlas2^%u|blas2^%u|px2^%u|spp2^%u|depth%u|images2^%u|bvh4%u",
+    std::snprintf(key, sizeof(key), "%s|features%u|tlas2^%u|blas2^%u|px2^%u|spp2^%u|depth%u|images2^%u|bvh4%u%s",
                   s->ctx->arch, s->features & 7u, log2_bucket(s->ds.tlas_len), log2_bucket(s->blas_len),
                   log2_bucket(pixels), log2_bucket(std::max(spp, 1u)), depth, log2_bucket(images),
-                  (flags & ORN_TUNE_ALLOW_BVH4) ? 1u : 0u);
+                  (flags & ORN_TUNE_ALLOW_BVH4) ? 1u : 0u,
+                  (s->features & kNoSearchTree) ? "|unordered" : "");  // other kernels, of twice the node visits
     return key;
 }
 
