@@ -1797,15 +1797,15 @@ static orn_status host_batch(orn_nrc *n, const orn_nrc_record *records, size_t c
     float l = 0.0f;
     static_assert(kMlpParams * 4 + 4 <= HostStage::kBytes, "gradient and loss fit the pinned buffer");
     char *pin = stage.pinned();
+    const bool want = !update && mlp_grad, staged = pin && (!want || HostStage::pageable(mlp_grad));
     float *h_loss = pin ? reinterpret_cast<float *>(pin) : &l;
-    float *h_grad = pin ? h_loss + 1 : mlp_grad;
-    const bool want = !update && mlp_grad;
+    float *h_grad = staged ? h_loss + 1 : mlp_grad;
     if (!e) e = hipMemcpyAsync(h_loss, n->loss, 4, hipMemcpyDeviceToHost, st);
     if (!e && want) e = hipMemcpyAsync(h_grad, n->mlp_grad, kMlpParams * 4, hipMemcpyDeviceToHost, st);
     const hipError_t w = hipStreamSynchronize(st);
     if (!e) e = w;
     if (e) return from_hip(e);
-    if (want && pin) std::memcpy(mlp_grad, h_grad, kMlpParams * 4);
+    if (want && staged) std::memcpy(mlp_grad, h_grad, kMlpParams * 4);
     if (loss) *loss = *h_loss;
     return ORN_OK;
 }

@@ -2652,7 +2652,7 @@ static orn_status trace_rays(orn_device_scene *s, float t_min, const float *rays
     static_assert(kRaysPerPiece * kRay <= HostStage::kPart && kRaysPerPiece % kBlock == 0,
                   "a piece of rays fits its part of the buffer");
     std::lock_guard<std::mutex> lock(ctx->stage.mutex);
-    if (n <= kDirectRays && ctx->stage.pinned()) {
+    if (n <= kDirectRays && HostStage::pageable(rays) && HostStage::pageable(out) && ctx->stage.pinned()) {
         float *h_rays = reinterpret_cast<float *>(ctx->stage.pinned());
         orn_hit *h_out = reinterpret_cast<orn_hit *>(ctx->stage.pinned() + kDirectRays * kRay);
         std::memcpy(h_rays, rays, n * kRay);

@@ -8,7 +8,9 @@
 // destination: 33 MB in 0.88 ms, a million rays and their hits 4.1 -> 3.1 ms,
 // a 1080p radiance-cache frame with its framebuffer 2.7 -> 1.8 ms, 500x500 at
 // 1 spp 0.51 -> 0.45 ms. One buffer per context, allocated by the first copy, freed
-// with the context.
+// with the context. Memory the runtime knows (pinned, managed, a device's) is
+// reached by the copy engines without it and may not be the host's to touch:
+// its copies go straight there.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -29,6 +31,15 @@ public:
     static constexpr size_t kPart = kBytes / kParts;
 
     std::mutex mutex;  // held for a whole call: the buffer has one user at a time
+
+    // Whether p is ordinary host memory.
+    static bool pageable(const void *p)
+    {
+        hipPointerAttribute_t a{};
+        if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+        (void)hipGetLastError();  // not known
+        return true;
+    }
 
     // The calls below need the mutex. Copies are ordered on `st` after the
     // work already there.
@@ -67,7 +78,7 @@ public:
     // Device to host; returns when dst is filled.
     hipError_t to_host(void *dst, const void *src, size_t bytes, int device, hipStream_t st)
     {
-        if (!pinned()) {
+        if (!pageable(dst) || !pinned()) {
             const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
             return e != hipSuccess ? e : hipStreamSynchronize(st);
         }
@@ -79,18 +90,20 @@ public:
         return hipSuccess;
     }
 
-    // Host to device in pieces of at most `piece` bytes (at most kPart); after(begin, bytes) enqueues what follows each piece. src may
-    // be reused on return; the buffer only after `st` has been waited for.
+    // Host to device in pieces of at most `piece` bytes (at most kPart);
+    // after(begin, bytes) enqueues what follows each piece. src and the buffer may
+    // be reused after `st` has been waited for.
     template <typename After>
     hipError_t to_device(void *dst, const void *src, size_t bytes, size_t piece, hipStream_t st, After after)
     {
         hipError_t e = hipSuccess;
+        const bool staged = pageable(src) && pinned();
         size_t i = 0;
         for (size_t at = 0; at < bytes && e == hipSuccess; at += piece, i++) {
             const size_t n = std::min(piece, bytes - at);
             const char *from = static_cast<const char *>(src) + at;
-            if (char *p = pinned()) {
-                p += (i % kParts) * kPart;
+            if (staged) {
+                char *p = pin_ + (i % kParts) * kPart;
                 if (i >= kParts) e = hipEventSynchronize(events_[i % kParts]);
                 if (e == hipSuccess) {
                     std::memcpy(p, from, n);
