@@ -1657,7 +1657,8 @@ void fill_sphere_leaves(const orn_scene_desc *d, std::vector<orn_bvh_node> &node
 // the cull (sphere_cull), and instances' boxes cull nothing.
 class SearchTree {
 public:
-    std::vector<uint32_t> nodes;  // TLAS trees, then BLAS trees, in the given format
+    std::vector<uint32_t> nodes;  // TLAS trees in the given format,
+    std::vector<uint32_t> blas_nodes;  // and the BLAS trees, which go behind them
     std::vector<uint32_t> roots;  // search root reference of each TLAS root
     uint32_t slots = 1;           // traversal stack entries it needs, in any order of the children
     SphereCull cull{};            // of a scene without meshes
@@ -1669,11 +1670,11 @@ public:
     {
         if (!nested(d->tlas_nodes, d->tlas_nodes_len) || !nested(d->blas_nodes, d->blas_nodes_len)) return false;
         std::vector<orn_bvh_node> t = tlas;
-        std::vector<uint32_t> b;  // the BLAS trees, from place 0 until they join the TLAS's
+        std::vector<uint32_t> &b = blas_nodes;  // from place 0 until all TLAS trees are known
         std::vector<uint32_t> blas_root(d->blas_nodes_len, kEmptyRef), blas_slots(d->blas_nodes_len, 0u);
         std::vector<MeshCore> core(d->blas_nodes_len);
         std::vector<orn_sah::Leaf> leaves, blas_leaves;
-        std::vector<uint32_t> below(t.size(), 0u);  // stack entries a TLAS leaf's BLAS needs
+        std::vector<uint32_t> blas_of(t.size(), 0u);  // stack entries a TLAS leaf's BLAS needs
         size_t collected = 0;
         for (size_t i = 0; i < n_roots; i++) {
             leaves.clear();
@@ -1706,12 +1707,12 @@ public:
                 nd.rmax_or_v3[2] = kEtaFar * core[r].eta * core[r].size;
                 l.ref = kLeafRef | static_cast<uint32_t>(t.size());
                 t.push_back(nd);
-                below.push_back(1u + blas_slots[r]);
+                blas_of.push_back(1u + blas_slots[r]);
             }
             uint32_t root = kEmptyRef;
             if (!grow(leaves, nodes, &root)) return false;
             roots.push_back(root);
-            slots = std::max(slots, pending(nodes, root, &below));
+            slots = std::max(slots, pending(nodes, root, &blas_of));
         }
         if (slots > kMaxStack || t.size() >= kLeafRef || (nodes.size() + b.size()) * 4u > 0xffffff00ull)
             return false;
@@ -1724,7 +1725,6 @@ public:
             move(b[at + right_at()]);
         }
         for (size_t i = d->tlas_nodes_len; i < t.size(); i++) move(t[i].left_or_custom_id);  // mesh leaves' copies
-        nodes.insert(nodes.end(), b.begin(), b.end());
         tlas = std::move(t);
         return true;
     }
@@ -1849,7 +1849,7 @@ private:
     static MeshCore mesh_core(const orn_bvh_node *n, const std::vector<orn_sah::Leaf> &triangles)
     {
         constexpr int kKappas[] = {6, 8, 10, 12};  // kappa 2^-6 to 2^-12
-        constexpr int kRays = 256;                 // that the cores are compared over
+        constexpr int kRays = 64;                  // that the cores are compared over
         constexpr double kFar = 64.0;              // mesh sizes between an open mesh and its core's centre
         auto dot3 = [](const double *x, const double *y) { return x[0] * y[0] + x[1] * y[1] + x[2] * y[2]; };
         auto cross3 = [](const double *x, const double *y, double *z) {
@@ -1881,31 +1881,34 @@ private:
         MeshCore best;
         int met = 0;  // rays that reach its ball
         auto consider = [&](const float *centre) {
-            double radius[4], least_sine = 1.0, size = 0.0;
-            if (!core_radii(n, triangles, centre, kKappas, radius, &least_sine, &size)) return;
-            const double u = kUnit, tau = 20.2 * u / least_sine;
-            for (int k = 0; k < 4; k++) {
-                const double eta = 10.3 * u * std::ldexp(1.0, kKappas[k]), r = radius[k] - tau * size;
+            double pass2[kRays], from2[kRays];  // squared distances of rays through points of the mesh, and of those
+            uint32_t seed = 1u;
+            auto draw = [&seed] {
+                seed = seed * 1664525u + 1013904223u;
+                return double(seed >> 8) / 16777216.0;
+            };
+            for (int i = 0; i < kRays; i++) {
+                const orn_bvh_node &nd = n[triangles[size_t(draw() * double(triangles.size()))].ref & ~kLeafRef];
+                const double z = 2.0 * draw() - 1.0, phi = 6.283185307179586 * draw(), ring = std::sqrt(1.0 - z * z);
+                const double d[3] = {ring * std::cos(phi), ring * std::sin(phi), z};
+                double p[3], off[3];
+                for (int a = 0; a < 3; a++)
+                    p[a] = (double(nd.lmin_or_v0[a]) + nd.lmax_or_v1[a] + nd.rmin_or_v2[a]) / 3.0 - centre[a];
+                cross3(p, d, off);
+                pass2[i] = dot3(off, off);
+                from2[i] = dot3(p, p);
+            }
+            // a smaller kappa widens every cull fourfold: for an eighth more rays only
+            for (int k = 0; k < 4 && met < kRays - kRays / 8; k++) {
+                double least_sine = 1.0, size = 0.0;
+                const double kappa = std::ldexp(1.0, -kKappas[k]);
+                const double radius = core_radius(n, triangles, centre, kappa, &least_sine, &size);
+                const double u = kUnit, eta = 10.3 * u / kappa, tau = 20.2 * u / least_sine, r = radius - tau * size;
                 // the test on the device leaves eta / kEtaBall of the origin's distance for its rounding and tau
-                if (30.0 * u + 1.01 * tau > eta / kEtaBall || !(r >= kLeastLength && r <= kMostLength)) continue;
+                if (30.0 * u + 1.01 * tau > eta / kEtaBall || !(r >= kLeastLength && size <= kMostLength)) continue;
                 const double r2 = r * r * (1.0 - tau) * (1.0 - 16.0 * u);
-                uint32_t seed = 1u;  // rays through points of the mesh, in any direction
-                auto draw = [&seed] {
-                    seed = seed * 1664525u + 1013904223u;
-                    return double(seed >> 8) / 16777216.0;
-                };
                 int count = 0;
-                for (int i = 0; i < kRays; i++) {
-                    const orn_bvh_node &nd = n[triangles[size_t(draw() * double(triangles.size()))].ref & ~kLeafRef];
-                    const double z = 2.0 * draw() - 1.0, phi = 6.283185307179586 * draw(), ring = std::sqrt(1.0 - z * z);
-                    const double d[3] = {ring * std::cos(phi), ring * std::sin(phi), z};
-                    double p[3], off[3];
-                    for (int a = 0; a < 3; a++)
-                        p[a] = (double(nd.lmin_or_v0[a]) + nd.lmax_or_v1[a] + nd.rmin_or_v2[a]) / 3.0 - centre[a];
-                    cross3(p, d, off);
-                    count += dot3(off, off) + eta / kEtaBall * dot3(p, p) < r2;
-                }
-                // a smaller kappa widens every cull fourfold: for an eighth more rays only
+                for (int i = 0; i < kRays; i++) count += pass2[i] + eta / kEtaBall * from2[i] < r2;
                 if (count <= met + kRays / 8) continue;
                 met = count;
                 for (int a = 0; a < 3; a++) best.centre[a] = centre[a];
@@ -1921,15 +1924,15 @@ private:
 
     static constexpr double kLeastLength = 1e-12, kMostLength = 1e12;  // products neither under- nor overflow
 
-    // The ball's radius for each kappa 2^-k, the least sine of an angle at a first
-    // vertex and the farthest vertex. False if a mesh can have no core.
-    static bool core_radii(const orn_bvh_node *n, const std::vector<orn_sah::Leaf> &triangles, const float *centre,
-                           const int (&kappas)[4], double (&radius)[4], double *least_sine, double *size)
+    // The ball's radius for a kappa (negative: none), the least sine of an angle
+    // at a first vertex and the farthest vertex.
+    static double core_radius(const orn_bvh_node *n, const std::vector<orn_sah::Leaf> &triangles, const float *centre,
+                              double kappa, double *least_sine, double *size)
     {
-        std::fill(radius, radius + 4, std::numeric_limits<double>::infinity());
+        double radius = std::numeric_limits<double>::infinity(), far2 = 0.0;
         for (const orn_sah::Leaf &l : triangles) {
             const orn_bvh_node &nd = n[l.ref & ~kLeafRef];
-            double v[3][3], e1[3], e2[3], far2 = 0.0, l1 = 0.0, l2 = 0.0, area = 0.0, h = 0.0;
+            double v[3][3], e1[3], e2[3], l1 = 0.0, l2 = 0.0, area2 = 0.0, h = 0.0;
             for (int a = 0; a < 3; a++) {
                 v[0][a] = double(nd.lmin_or_v0[a]) - centre[a];
                 v[1][a] = double(nd.lmax_or_v1[a]) - centre[a];
@@ -1940,28 +1943,22 @@ private:
                 l2 += e2[a] * e2[a];
             }
             for (const auto &p : v) far2 = std::max(far2, p[0] * p[0] + p[1] * p[1] + p[2] * p[2]);
-            *size = std::max(*size, std::sqrt(far2));
             if (l1 == 0.0 || l2 == 0.0) continue;  // its determinant is 0 and its t NaN: never hit
-            l1 = std::sqrt(l1);
-            l2 = std::sqrt(l2);
             for (int a = 0; a < 3; a++) {
                 const double c = e1[(a + 1) % 3] * e2[(a + 2) % 3] - e1[(a + 2) % 3] * e2[(a + 1) % 3];
-                area += c * c;
+                area2 += c * c;
                 h += c * v[0][a];
             }
-            area = std::sqrt(area);
-            const double sine = area / (l1 * l2);
-            if (!(std::min(l1, l2) >= kLeastLength) || !(sine > 0.0)) return false;
-            h = std::fabs(h) / area;
+            const double sine = std::sqrt(area2 / (l1 * l2)), x = 2.0 * kappa / (sine * sine);
+            if (!(std::min(l1, l2) >= kLeastLength * kLeastLength) || !(x <= 0.7)) return -1.0;
+            const double h2 = h * h / area2, v2 = v[0][0] * v[0][0] + v[0][1] * v[0][1] + v[0][2] * v[0][2];
             *least_sine = std::min(*least_sine, sine);
-            const double w = std::sqrt(std::max(0.0, v[0][0] * v[0][0] + v[0][1] * v[0][1] + v[0][2] * v[0][2] - h * h));
-            for (int k = 0; k < 4; k++) {
-                const double kappa = std::ldexp(1.0, -kappas[k]), x = 2.0 * kappa / (sine * sine);
-                const double r = x > 0.7 ? -1.0 : h * std::sqrt(1.0 - x * x) - x * w - 2.1 * kappa * std::max(l1, l2) / sine;
-                radius[k] = std::min(radius[k], r);
-            }
+            radius = std::min(radius, std::sqrt(h2 * (1.0 - x * x)) - x * std::sqrt(std::max(0.0, v2 - h2)) -
+                                          2.1 * kappa * std::sqrt(std::max(l1, l2)) / sine);
+            if (!(radius >= kLeastLength)) return -1.0;
         }
-        return *size <= kMostLength;
+        *size = std::sqrt(far2);
+        return radius;
     }
 
     // The leaves below `root` with the boxes their parents hold for them (a
@@ -1969,6 +1966,7 @@ private:
     static void collect(const orn_bvh_node *n, uint32_t root, std::vector<orn_sah::Leaf> &out)
     {
         std::vector<uint32_t> todo;
+        out.reserve(root / 2u + 1u);  // parents follow their children
         auto visit = [&](uint32_t i, const orn_sah::Box &b) {
             if (n[i].node_type == 0u) todo.push_back(i);
             else out.push_back({b, kLeafRef | i});
@@ -2107,7 +2105,6 @@ orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots
     {
         auto flag = [](const orn_bvh_node *arr, uint32_t i) { return arr[i].node_type != 0u ? (i | kLeafRef) : i; };
         std::vector<orn_bvh_node> t2(desc->tlas_nodes, desc->tlas_nodes + desc->tlas_nodes_len);
-        std::vector<orn_bvh_node> b2(desc->blas_nodes, desc->blas_nodes + desc->blas_nodes_len);
         for (orn_bvh_node &nd : t2) {
             if (nd.node_type == 0u) {
                 nd.left_or_custom_id = flag(desc->tlas_nodes, nd.left_or_custom_id);
@@ -2116,11 +2113,6 @@ orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots
                 nd.left_or_custom_id = flag(desc->blas_nodes, nd.left_or_custom_id);
             }
         }
-        for (orn_bvh_node &nd : b2)
-            if (nd.node_type == 0u) {
-                nd.left_or_custom_id = flag(desc->blas_nodes, nd.left_or_custom_id);
-                nd.right_or_material_index = flag(desc->blas_nodes, nd.right_or_material_index);
-            }
         for (size_t i = 0; i < n_roots; i++) root2[i] = flag(desc->tlas_nodes, roots[i]);
         ds.tlas2_root = root2[0];
         ds.plain_spheres = spheres_are_plain(desc) ? 1u : 0u;
@@ -2136,23 +2128,32 @@ orn_status upload_scene(orn_ctx *ctx, const orn_scene_desc *desc, uint32_t slots
         if (!ordered) s->features |= kNoSearchTree;
         s->traversal_slots = ordered ? std::max(slots, search.slots) : slots;
         ds.cull = search.cull;
-        // one array: the BLAS nodes behind the TLAS's
-        const size_t tlas_n = t2.size();
-        if (tlas_n + b2.size() >= kLeafRef) return fail(ORN_ERROR_OUT_OF_MEMORY);
+        // one array: the search tree in front (the two are read in turn), the BLAS
+        // nodes behind the TLAS's
+        const size_t tlas_n = t2.size(), blas_n = desc->blas_nodes_len;
+        if (tlas_n + blas_n >= kLeafRef) return fail(ORN_ERROR_OUT_OF_MEMORY);
         const uint32_t shift = static_cast<uint32_t>(tlas_n);  // leaves the flag alone
         for (size_t i = 0; i < desc->tlas_nodes_len; i++)  // (the search tree's copies have their own roots)
             if (t2[i].node_type == 2u) t2[i].left_or_custom_id += shift;
-        for (orn_bvh_node &nd : b2)
+        const size_t words = ordered ? search.nodes.size() + search.blas_nodes.size() : 0, ahead = (words + 15) / 16;
+        std::vector<orn_bvh_node> all;
+        all.reserve(ahead + tlas_n + blas_n);
+        all.resize(ahead);
+        if (words) {
+            char *const at = reinterpret_cast<char *>(all.data());
+            std::memcpy(at, search.nodes.data(), 4 * search.nodes.size());
+            std::memcpy(at + 4 * search.nodes.size(), search.blas_nodes.data(), 4 * search.blas_nodes.size());
+        }
+        all.insert(all.end(), t2.begin(), t2.end());
+        for (size_t i = 0; i < blas_n; i++) {
+            orn_bvh_node nd = desc->blas_nodes[i];
             if (nd.node_type == 0u) {
-                nd.left_or_custom_id += shift;
-                nd.right_or_material_index += shift;
+                nd.left_or_custom_id = flag(desc->blas_nodes, nd.left_or_custom_id) + shift;
+                nd.right_or_material_index = flag(desc->blas_nodes, nd.right_or_material_index) + shift;
             }
-        t2.insert(t2.end(), b2.begin(), b2.end());
-        // and the search tree in front of it (one allocation: the two are read in turn)
-        const size_t ahead = ordered ? (search.nodes.size() + 15) / 16 : 0;
-        t2.insert(t2.begin(), ahead, orn_bvh_node{});
-        if (ordered) std::memcpy(t2.data(), search.nodes.data(), 4 * search.nodes.size());
-        if ((st = upload(s, reinterpret_cast<const float4 *>(t2.data()), 4 * t2.size(), &f4))) return fail(st);
+            all.push_back(nd);
+        }
+        if ((st = upload(s, reinterpret_cast<const float4 *>(all.data()), 4 * all.size(), &f4))) return fail(st);
         ds.search = ordered ? reinterpret_cast<const char *>(f4) : nullptr;
         ds.nodes2 = f4 + 4 * ahead;
         ds.blas2 = ds.nodes2 + 4 * tlas_n;
