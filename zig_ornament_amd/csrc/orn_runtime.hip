@@ -1671,10 +1671,14 @@ public:
         if (!nested(d->tlas_nodes, d->tlas_nodes_len) || !nested(d->blas_nodes, d->blas_nodes_len)) return false;
         std::vector<orn_bvh_node> t = tlas;
         std::vector<uint32_t> &b = blas_nodes;  // from place 0 until all TLAS trees are known
-        std::vector<uint32_t> blas_root(d->blas_nodes_len, kEmptyRef), blas_slots(d->blas_nodes_len, 0u);
-        std::vector<MeshCore> core(d->blas_nodes_len);
+        struct Blas {
+            uint32_t root, slots;
+            MeshCore core;
+        };
+        std::vector<Blas> blases;
+        std::vector<uint32_t> blas_at(d->blas_nodes_len, kEmptyRef);  // of a BLAS root, in `blases`
         std::vector<orn_sah::Leaf> leaves, blas_leaves;
-        std::vector<uint32_t> blas_of(t.size(), 0u);  // stack entries a TLAS leaf's BLAS needs
+        std::vector<uint32_t> below(t.size(), 0u);  // stack entries a TLAS leaf's BLAS needs
         size_t collected = 0;
         for (size_t i = 0; i < n_roots; i++) {
             leaves.clear();
@@ -1691,28 +1695,31 @@ public:
                     continue;
                 }
                 const uint32_t r = d->tlas_nodes[idx].left_or_custom_id;
-                if (blas_root[r] == kEmptyRef) {
+                if (blas_at[r] == kEmptyRef) {
                     blas_leaves.clear();
                     collect(d->blas_nodes, r, blas_leaves);
                     collected += blas_leaves.size();
                     if (collected > 2 * d->blas_nodes_len) return false;  // roots inside one another's trees
-                    core[r] = mesh_core(d->blas_nodes, blas_leaves);
-                    if (!grow(blas_leaves, b, &blas_root[r])) return false;
-                    blas_slots[r] = pending(b, blas_root[r], nullptr);
+                    Blas made{kEmptyRef, 0u, mesh_core(d->blas_nodes, blas_leaves)};
+                    if (!grow(blas_leaves, b, &made.root)) return false;
+                    made.slots = pending(b, made.root, nullptr);
+                    blas_at[r] = static_cast<uint32_t>(blases.size());
+                    blases.push_back(made);
                 }
-                nd.left_or_custom_id = blas_root[r];
-                std::memcpy(nd.rmin_or_v2, core[r].centre, 12);  // more words not otherwise read
-                nd.rmax_or_v3[0] = core[r].radius2;
-                nd.rmax_or_v3[1] = kEtaNear * core[r].eta;
-                nd.rmax_or_v3[2] = kEtaFar * core[r].eta * core[r].size;
+                const Blas &blas = blases[blas_at[r]];
+                nd.left_or_custom_id = blas.root;
+                std::memcpy(nd.rmin_or_v2, blas.core.centre, 12);  // more words not otherwise read
+                nd.rmax_or_v3[0] = blas.core.radius2;
+                nd.rmax_or_v3[1] = kEtaNear * blas.core.eta;
+                nd.rmax_or_v3[2] = kEtaFar * blas.core.eta * blas.core.size;
                 l.ref = kLeafRef | static_cast<uint32_t>(t.size());
                 t.push_back(nd);
-                blas_of.push_back(1u + blas_slots[r]);
+                below.push_back(1u + blas.slots);
             }
             uint32_t root = kEmptyRef;
             if (!grow(leaves, nodes, &root)) return false;
             roots.push_back(root);
-            slots = std::max(slots, pending(nodes, root, &blas_of));
+            slots = std::max(slots, pending(nodes, root, &below));
         }
         if (slots > kMaxStack || t.size() >= kLeafRef || (nodes.size() + b.size()) * 4u > 0xffffff00ull)
             return false;
