@@ -42,6 +42,17 @@ def wall_mesh(n):
     return verts[:one], tris[: 6 * n * n]
 
 
+def ring_mesh(n, m):
+    """A torus: triangle planes of it pass through its middle."""
+    a, b = np.meshgrid(2 * np.pi * np.arange(n) / n, 2 * np.pi * np.arange(m) / m, indexing="ij")
+    r = 1.0 + 0.4 * np.cos(b)
+    verts = np.stack([r * np.cos(a), 0.4 * np.sin(b), r * np.sin(a), np.ones_like(a)], -1).reshape(-1, 4)
+    i, j = np.meshgrid(np.arange(n), np.arange(m), indexing="ij")
+    k00, k01 = i * m + j, i * m + (j + 1) % m
+    k10, k11 = (i + 1) % n * m + j, (i + 1) % n * m + (j + 1) % m
+    return verts.astype(np.float32), np.stack([k00, k01, k11, k00, k11, k10], -1).reshape(-1).astype(np.uint32)
+
+
 def mesh_spec(mesh, count, box, seed):
     """Instances of a mesh, scaled, turned any way and placed in a box."""
     rng = np.random.default_rng(seed)
@@ -137,6 +148,8 @@ MESHES = {
     "boxes": lambda: mesh_spec(box_mesh(1), 2000, 20.0, 2),
     "tiles": lambda: mesh_spec(box_mesh(6), 300, 20.0, 3),      # flat faces of many triangles
     "walls": lambda: mesh_spec(wall_mesh(4), 400, 16.0, 4),     # open: the core lies in front of them
+    "ring": lambda: mesh_spec(ring_mesh(24, 12), 3, 3.0, 6),    # no core: searched whole
+    "rings": lambda: mesh_spec(ring_mesh(24, 12), 60, 9.0, 7),  # many of them: the reference's order
     "balls": lambda: mesh_spec(W.icosphere_mesh(3)[:2], 200, 12.0, 5),
 }
 

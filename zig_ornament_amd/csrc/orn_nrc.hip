@@ -43,7 +43,7 @@ constexpr uint32_t kBlock = 256;
 // Internal BVH nodes a lane visits in a row before a leaf visit (bvh_hit). The
 // nearest-first search reaches a leaf after few nodes, and lanes there wait
 // out the rest of the run: 1, 2, 3, 4, 6, 8 and 16 nodes give a frame over the
-// 1,024 icospheres 0.835, 0.80, 0.825, 0.823, 0.823, 0.836 and 0.89 ms, one
+// 1,024 icospheres 0.97, 0.925, 0.94, 0.945, 0.955, 0.98 and 1.03 ms, one
 // over spheres 1.45-1.47 ms throughout.
 constexpr uint32_t kNodeSteps = 2;
 // nrc_grid_kernel: table entries per workgroup (64 KB of LDS, two feature

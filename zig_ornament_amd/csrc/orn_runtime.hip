@@ -776,12 +776,11 @@ __global__ __launch_bounds__(kBlock) void post_batch_kernel(const BatchItem *__r
 // kHeavyLanes each (render_kernel). One wave per band.
 // Why: a pixel is one lane's work, so a launch takes at least the time of its
 // costliest one, and in a full wave every step of that pixel waits for 63
-// other lanes' node, leaf and shading rounds. Where that is what binds (1,024
-// instanced icospheres 1080p, 32 spp: the launch 20.6 ms, its costliest pixel
-// 20.5, all pixels spread evenly over the lanes 15), the few pixels above both
-// an even share and half of the costliest run at half the time in waves of 4:
-// 20.6 -> 18.4 ms; an instanced scene of 490,000 pixels, 8 spp 3.75 -> 3.37; 16
-// images of 630,000 pixels 9.5 (in tile order; ordered before 9.9) -> 6.45.
+// other lanes' node, leaf and shading rounds. Where that is what binds, the few
+// pixels above both an even share and half of the costliest run at half the time
+// in waves of 4: 1,024 instanced icospheres 1080p, 32 spp, ordered by cost 26.5 ->
+// 22.6 ms; an instanced scene of 490,000 pixels, 8 spp 4.4 -> 3.7; 16 images of
+// 630,000 pixels 10.6 -> 6.85.
 // Random spheres 1080p, 64 spp, has no such pixels and keeps its 23.2. Waves of 2 to
 // 8 heavy lanes, shares of a half or a quarter and parts of 0.4 to 0.6 differ by less
 // than 2 %; 16 lanes cost 4 %, and no limit on the share 15 %.
@@ -1302,12 +1301,12 @@ orn_tuning default_tuning()
 // did best over 12 images (random spheres, icospheres, Cornell boxes, 250,000
 // to 2 million pixels, 1 to 64 spp, as a geometric mean over 55 shapes): 7 %
 // less time than default_tuning(), 11 % with queues by cost. Those pay once
-// pixels are long (2000x1000, 15 spp 6.8 -> 6.35 ms; random spheres 1080p 64 spp
-// 29.9 -> 24.3; but 1080p 4 spp 2.49 -> 2.46, 500x500 1 spp 0.240 -> 0.258) and
+// pixels are long (2000x1000, 15 spp 6.55 -> 6.2 ms; random spheres 1080p 64 spp
+// 28.2 -> 23.5; but 1080p 4 spp 2.46 -> 2.44, 500x500 1 spp 0.227 -> 0.248) and
 // many enough for the lanes to take more than one or for heavy pixels to have
 // lanes to spare (8 spp, plain -> ordered first -> later: instanced scenes 256x256
-// 1.87 -> 1.96 -> 1.91 ms, 512x512 2.22 -> 2.09 -> 1.99; Cornell boxes 0.77 -> 0.97
-// -> 0.81 and 1.20 -> 1.35 -> 1.11). A batch records its costs as it goes, so its
+// 1.94 -> 2.31 -> 1.70 ms, 512x512 2.46 -> 2.17 -> 1.93; Cornell boxes 0.78 -> 0.98
+// -> 0.82 and 1.17 -> 1.32 -> 1.09). A batch records its costs as it goes, so its
 // first render costs nothing more (131,072 to 1 million pixels of 1 to 32 spp: first
 // within 5 % of plain, later 5 to 30 % less; 32,768 pixels 1.15 -> 1.28).
 constexpr uint32_t kCostOrderSpp = 8, kCostOrderPixels = 1u << 17;
@@ -1423,10 +1422,10 @@ hipError_t launch_render_k(uint32_t per_cu, uint32_t cus, size_t lds, hipStream_
     // tuning may launch more workgroups than fit: those run when the pixels are
     // gone, and counting their lanes left the others sparse: random spheres 500x500,
     // 8 spp, in 32 workgroups per CU 2.68 ms, now 1.07.)
-    // 8 spp, full -> sparse: instanced icospheres 64x64 1.64 -> 0.92 ms,
-    // 160x160 1.91 -> 1.36; random spheres 128x128 0.97 -> 0.75, 160x160 0.94 ->
-    // 0.85; Cornell box (every path bounces to its full depth) 96x96 0.86 ->
-    // 0.65, 181x181 0.85 -> 0.87. Above that the box loses more than the others
+    // 8 spp, full -> sparse: instanced icospheres 64x64 1.59 -> 1.03 ms,
+    // 160x160 1.80 -> 1.32; random spheres 128x128 0.90 -> 0.70, 160x160 0.92 ->
+    // 0.81; Cornell box (every path bounces to its full depth) 96x96 0.76 ->
+    // 0.65, 181x181 0.77 -> 0.82. Above that the box loses more than the others
     // gain (200x200 at 12 lanes: 0.83 -> 0.96, icospheres 1.83 -> 1.50).
     KernelParams kp = a.kp;
     const uint32_t per_wave = blocks_for(kp.pixels, resident * (kBlock / 64u));
@@ -1651,7 +1650,8 @@ void fill_sphere_leaves(const orn_scene_desc *d, std::vector<orn_bvh_node> &node
 // Rays get the reference's hits only if its boxes are what its build makes
 // them: finite, each containing the boxes below it, a triangle's own spanning
 // its vertices, every node under one parent. Arrays that are not so keep the
-// reference's order throughout (build returns false and leaves them alone).
+// reference's order throughout (build returns false and leaves them alone), and
+// so do scenes that are no faster for the search (kCoreless).
 // A sphere's box need not hold the sphere, nor an instance's box its mesh
 // (transforms moved under kept boxes): what a sphere's box leaves out widens
 // the cull (sphere_cull), and instances' boxes cull nothing.
@@ -1679,7 +1679,7 @@ public:
         std::vector<uint32_t> blas_at(d->blas_nodes_len, kEmptyRef);  // of a BLAS root, in `blases`
         std::vector<orn_sah::Leaf> leaves, blas_leaves;
         std::vector<uint32_t> below(t.size(), 0u);  // stack entries a TLAS leaf's BLAS needs
-        size_t collected = 0;
+        size_t collected = 0, instances = 0, coreless = 0;
         for (size_t i = 0; i < n_roots; i++) {
             leaves.clear();
             collect(d->tlas_nodes, tlas_roots[i], leaves);
@@ -1707,6 +1707,8 @@ public:
                     blases.push_back(made);
                 }
                 const Blas &blas = blases[blas_at[r]];
+                instances++;
+                coreless += blas.core.radius2 < 0.0f;
                 nd.left_or_custom_id = blas.root;
                 std::memcpy(nd.rmin_or_v2, blas.core.centre, 12);  // more words not otherwise read
                 nd.rmax_or_v3[0] = blas.core.radius2;
@@ -1721,6 +1723,7 @@ public:
             roots.push_back(root);
             slots = std::max(slots, pending(nodes, root, &below));
         }
+        if (coreless >= kCoreless && 2 * coreless > instances) return false;
         if (slots > kMaxStack || t.size() >= kLeafRef || (nodes.size() + b.size()) * 4u > 0xffffff00ull)
             return false;
         // the BLAS trees move behind the TLAS's, and BLAS leaves behind the TLAS nodes
@@ -1737,6 +1740,14 @@ public:
     }
 
 private:
+    // From so many instances of meshes without a core on, if they are most, rays
+    // take the reference's order: they would search each of them whole, and in
+    // that order a near hit still culls those behind it. Renders 960x540, 8 spp,
+    // reference's order against search tree: tori of 3,600 triangles x1000 38.6
+    // and 53.3 ms, x200 22.2 and 29.3, x16 10.6 and 13.0, x4 5.0 and 5.5, x2 4.2 and
+    // 4.3, one of 40,000 triangles 5.2 and 3.4 (x8 18.1 and 17.0, x200 39.1 and 42.5);
+    // 2,000 loose triangles x200 46 and 68, x4 14.0 and 16.4, x1 9.0 and 8.0.
+    static constexpr size_t kCoreless = 4;
     // Levels a search tree may be higher than the balanced one: enough for
     // the SAH's splits (random spheres and icospheres take 1 or 2), and the
     // stack it bounds stays close to the reference's.
@@ -2512,10 +2523,11 @@ orn_status orn_render_noalloc(orn_device_scene *s, const orn_constant_params *pa
     next_epoch();
     // There is no earlier call to take costs from, so an order by cost comes
     // from the call's own first eighth, as in a target's first render: 1,024
-    // instanced icospheres 1080p, 32 spp, 25.3 ms in tile order, 21.9 in jobs of
-    // two samples, 20.6 by cost; random spheres 64 spp 28.1 -> 25.7. Small
-    // images do not repay the second launch (see kCostOrderPixels), some
-    // larger ones neither (a Cornell box 512x512, 8 spp 1.18 -> 1.31), so only a
+    // instanced icospheres 1080p, 32 spp, 31.4 ms in tile order, 25.7 in jobs of
+    // two samples, 26.0 by cost; random spheres 64 spp 28.1, 38.1 and 25.8; textured
+    // icospheres 700x700, 8 spp 4.35, 4.23 and 4.04. Small images do not repay the
+    // second launch (see kCostOrderPixels), some larger ones neither (a Cornell
+    // box 512x512, 8 spp 1.21 -> 1.32), so only a
     // tuning that asks for it gets it. Split pixels keep tile order: they end
     // together without it.
     const bool whole = tn.split_percent == 0u || tn.samples_per_job == 0u || tn.samples_per_job >= iterations;

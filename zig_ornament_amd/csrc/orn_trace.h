@@ -265,8 +265,9 @@ enum SceneFeatures : uint32_t {
 // Node format of a BVH2 launch (the W of the traversal below). The wider nodes
 // of format 2 take a quarter more of the caches for their shorter test: random
 // spheres 1920x1080, 64 spp, 23.8 -> 23.3 ms with them and 500x500, 1 spp, 0.25 ->
-// 0.235 ms, but 1,024 instanced icospheres 20.4 -> 20.9 ms (cost-ordered, 32 spp; a
-// stride of 96 bytes 21.1, of 128 bytes 22.1). So the trees of a mesh scene,
+// 0.235 ms, but 1,024 instanced icospheres 20.4 -> 20.9 ms (cost-ordered, 32 spp,
+// with fewer visits, by a cull at every box; a stride of 96 bytes 21.1, of 128
+// bytes 22.1). So the trees of a mesh scene,
 // which are the large ones, keep the 64-byte boxes.
 constexpr uint32_t bvh2_format(uint32_t f) { return (f & kNoSearchTree) ? 1u : (f & kHasMeshes) ? 3u : 2u; }
 constexpr bool is_search_format(uint32_t w) { return w == 2u || w == 3u; }
@@ -309,13 +310,13 @@ constexpr bool is_search_format(uint32_t w) { return w == 2u || w == 3u; }
 // The search is bound by the vector instructions of its node visits, so fewer
 // visits are time: random spheres 1920x1080, 64 spp, 52 -> 33 ms with it. The
 // kernels of mesh scenes in the reference's order and in this one: 1,024 instanced
-// icospheres 1080p, 32 spp, 33.5 -> 22.7 ms, textured, metal and glass icospheres
-// 700x700, 8 spp, 6.5 -> 3.76, 16 images of such scenes 9.7 -> 6.95, the Cornell
-// box 256x256, 16 spp, 1.58 -> 1.46, 200 tori (no core) 960x540, 8 spp, 32.2 -> 29.1.
-// (A cull by distance at every box would take the icospheres 18.5 ms and miss hits;
-// the instances behind the hit cost 2.1, the slack's arithmetic 0.9 and rays that
-// pass by the core 1.4.) Scenes whose arrays do not have nested boxes (SearchTree::build) have no search
-// tree.
+// icospheres 1080p, 32 spp, 33.7 -> 22.8 ms, textured, metal and glass icospheres
+// 700x700, 8 spp, 6.5 -> 3.75, 16 images of such scenes 9.5 -> 6.9, the Cornell
+// box 256x256, 16 spp, 1.52 -> 1.47, a radiance-cache frame over the icospheres
+// 1.25 -> 0.92. (A cull by distance at every box would take the icospheres 18.5 ms
+// and miss hits; the instances behind the hit cost 2.1, the slack's arithmetic 0.9
+// and rays that pass by the core 1.4.) Scenes whose arrays do not have nested
+// boxes, or which would not gain (SearchTree::build), have no search tree.
 struct Traversal {
     Ray ray;        // the ray in object space, inside a BLAS
     f3 inv, ox;     // safe_invdir(d) and -o * inv of the ray in the current space
